@@ -1,0 +1,64 @@
+/*
+ * qqt_learn.h - C ABI of the training kernels that work on whole parameter
+ * tensors (libqqt_hip.so, beside qqt_hip.h; same conventions: plain device
+ * pointers, asynchronous on the caller's stream, no allocation, 0 or a
+ * negative QQT_E_* code with qqt_last_error()).
+ */
+#ifndef QQT_LEARN_H
+#define QQT_LEARN_H
+
+#include <stdint.h>
+
+#ifdef __cplusplus
+extern "C" {
+#endif
+
+/* One PPO minibatch of the mlp ActorCritic above its first layer
+ * (train/ppo.py:401-421 on train/model.py:140-153, 192-196, 215-256): from
+ * z1 = x W0^T + b0 to the gradient of every parameter but W0, and dz1 for
+ * W0's (qqt_l1_grad).  The parameters are the module's own float32 tensors
+ * (contiguous); heads in the order move, bomb, critic with 5, 2 and 1
+ * outputs. */
+typedef struct qqt_ppo_step_args {
+  int32_t batch;              /* rows B (the means' divisor) */
+  float clip_eps;             /* float32(clip_eps): value clip and clip fraction */
+  float ratio_lo, ratio_hi;   /* float32(1 - clip_eps), float32(1 + clip_eps) */
+  float value_coef, entropy_coef;
+  int64_t workspace_bytes;
+  int64_t src_rows;           /* rows of the per-row inputs when row_index is set */
+  const int64_t* row_index;   /* [B] or NULL: actions, masks, old_logp, adv, ret and old_val
+                                 of row b are their row row_index[b], clamped into
+                                 [0, src_rows); z1 and dz1 stay in minibatch order */
+  const float* z1;            /* [B][128], 16-byte aligned */
+  const float *ln1_w, *ln1_b; /* [128] */
+  const float *w1, *b1;       /* [128][128], [128] */
+  const float *ln2_w, *ln2_b; /* [128] */
+  const float* wh[3];         /* [64][128] each */
+  const float* bh[3];         /* [64] each */
+  const float* wf[3];         /* [5][64], [2][64], [1][64] */
+  const float* bf[3];         /* [5], [2], [1] */
+  const int64_t* actions;     /* [.][2] */
+  const uint8_t* move_mask;   /* [.][5] */
+  const uint8_t* bomb_mask;   /* [.][2] */
+  const float *old_logp, *adv, *ret, *old_val;   /* [.] */
+  float* dz1;                 /* [B][128], 16-byte aligned */
+  float* dz_scale;            /* [1]: power of two that brings max |dz1| to about 2^14 */
+  float* stats;               /* [5]: pg, vf, entropy, old_logp - logp, clip fraction (means) */
+  float* db0;                 /* [128] column sums of dz1 */
+  float *dln1_w, *dln1_b, *dw1, *db1, *dln2_w, *dln2_b;
+  float* dwh[3];
+  float* dbh[3];
+  float* dwf[3];
+  float* dbf[3];
+  void* workspace;            /* qqt_ppo_step_workspace_bytes(B) bytes, 16-byte aligned */
+} qqt_ppo_step_args;
+
+/* Workspace of qqt_ppo_step for a batch (-1 for a bad batch). */
+int64_t qqt_ppo_step_workspace_bytes(int32_t batch);
+
+int qqt_ppo_step(const qqt_ppo_step_args* args, void* stream);
+
+#ifdef __cplusplus
+}
+#endif
+#endif /* QQT_LEARN_H */

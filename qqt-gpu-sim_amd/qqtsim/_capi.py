@@ -104,6 +104,18 @@ class PpoArgsC(ctypes.Structure):
                                                    ("row_index", _vp), ("src_rows", ctypes.c_int64)]
 
 
+class PpoStepArgsC(ctypes.Structure):
+    _fields_ = [("batch", _i32)] + [(n, _f32) for n in (
+        "clip_eps", "ratio_lo", "ratio_hi", "value_coef", "entropy_coef")] + [
+        ("workspace_bytes", ctypes.c_int64), ("src_rows", ctypes.c_int64)] + [
+        (n, _vp) for n in ("row_index", "z1", "ln1_w", "ln1_b", "w1", "b1", "ln2_w", "ln2_b")] + [
+        (n, _vp * 3) for n in ("wh", "bh", "wf", "bf")] + [
+        (n, _vp) for n in ("actions", "move_mask", "bomb_mask", "old_logp", "adv", "ret",
+                           "old_val", "dz1", "dz_scale", "stats", "db0", "dln1_w", "dln1_b",
+                           "dw1", "db1", "dln2_w", "dln2_b")] + [
+        (n, _vp * 3) for n in ("dwh", "dbh", "dwf", "dbf")] + [("workspace", _vp)]
+
+
 class CnnArgsC(ctypes.Structure):
     _fields_ = [(n, _i32) for n in (
         "batch", "npid", "pid0", "sample", "obs_stride", "mm_row_stride", "mm_pid_stride",
@@ -177,6 +189,10 @@ def lib():
         L.qqt_l1_grad_workspace_floats.argtypes = [_i32, _i32]
         L.qqt_ppo_grad.restype = ctypes.c_int
         L.qqt_ppo_grad.argtypes = [ctypes.POINTER(PpoArgsC), _vp]
+        L.qqt_ppo_step.restype = ctypes.c_int
+        L.qqt_ppo_step.argtypes = [ctypes.POINTER(PpoStepArgsC), _vp]
+        L.qqt_ppo_step_workspace_bytes.restype = ctypes.c_int64
+        L.qqt_ppo_step_workspace_bytes.argtypes = [_i32]
         L.qqt_cnn_act.restype = ctypes.c_int
         L.qqt_cnn_act.argtypes = [ctypes.POINTER(CnnArgsC), _vp]
         L.qqt_lstm_features.restype = ctypes.c_int

@@ -51,15 +51,6 @@ def _w0_fragments(w: torch.Tensor, kpad: int) -> torch.Tensor:
     return f.half().reshape(-1)
 
 
-def _kfrag(m: torch.Tensor) -> torch.Tensor:
-    """k-major [K][N] (multiples of 16) -> the MFMA fragments qqt_ppo_grad
-    reads: value i of lane 16 q + r in 16-k group g of column tile t is
-    M[16 g + 4 q + i][16 t + r]."""
-    k, n = m.shape
-    return (m.float().reshape(k // 16, 4, 4, n // 16, 16).permute(3, 0, 1, 4, 2)
-            .contiguous().reshape(-1))
-
-
 class _FirstLayer(torch.autograd.Function):
     @staticmethod
     def forward(ctx, x16, w0, b0, pid, owner):
@@ -114,8 +105,6 @@ def _lin(mod: nn.Linear, x):
 
 
 class HipMlpActorCritic(nn.Module):
-    GRAD_CHUNK = 4096       # rows per chunk of the batched weight-gradient products
-
     arch = "mlp"
 
     def __init__(self, obs_shape=(14, 13, 13), n_moves: int = 5, n_bomb: int = 2,
@@ -181,16 +170,18 @@ class HipMlpActorCritic(nn.Module):
         _capi.check(self._lib.qqt_mlp_act(a, _capi.stream_handle(x16.device)))
         return z1
 
-    def _l1_weight_grad(self, x16, dz1, pid, amax=None, rows=None):
-        """dW0 of the rows of x16 (or of its rows `rows`) against dz1; `amax`
-        = max |dz1| when the caller has it."""
+    def _l1_weight_grad(self, x16, dz1, pid, scale=None, rows=None):
+        """dW0 of the rows of x16 (or of its rows `rows`) against dz1; `scale`
+        (device, 1 value) = the power of two that brings max |dz1| to ~2^14
+        when the caller has it."""
         a = _capi.L1GradArgsC()
         b = self._rows_args(a, x16, rows)
         need = int(self._lib.qqt_l1_grad_workspace_floats(b, self.k0))
         if self._ws is None or self._ws.numel() < need:
             self._ws = torch.empty(need, dtype=torch.float32, device=x16.device)
-        amax = (dz1.abs().amax() if amax is None else amax).clamp_min(1e-30)
-        scale = torch.exp2(torch.clamp(14.0 - torch.ceil(torch.log2(amax)), -100.0, 100.0))
+        if scale is None:
+            amax = dz1.abs().amax().clamp_min(1e-30)
+            scale = torch.exp2(torch.clamp(14.0 - torch.ceil(torch.log2(amax)), -100.0, 100.0))
         dw0p = torch.empty((HID, self.k0), dtype=torch.float32, device=x16.device)
         a.batch, a.k0, a.obs_stride = b, self.k0, x16.stride(0)
         a.workspace_floats = self._ws.numel()
@@ -234,10 +225,9 @@ class HipMlpActorCritic(nn.Module):
         player 0's view) written into every parameter's `.grad`, as
         `loss.backward()` through `evaluate` would leave them; returns the
         five statistics (pg, vf, ent, kl, clipfrac) as a device tensor.
-        Three launches: the first layer's forward, `qqt_ppo_grad` (the loss
-        and the backward above the first layer) and `qqt_l1_grad`; the weight
-        gradients of the 128-wide layers are batched products of its row
-        outputs.  With `rows` (int64 indices), every per-row argument (obs,
+        Three calls: the first layer's forward, `qqt_ppo_step` (the loss, the
+        backward above the first layer and every gradient there) and
+        `qqt_l1_grad`.  With `rows` (int64 indices), every per-row argument (obs,
         masks, actions, old log-probs, advantages, returns, old values) is a
         whole buffer and the minibatch is its rows `rows`, which the kernels
         read in place."""
@@ -245,84 +235,58 @@ class HipMlpActorCritic(nn.Module):
         x16 = obs.reshape(obs.shape[0], -1)
         x16 = (x16 if x16.dtype == torch.float16 else x16.half()).contiguous()
         b = x16.shape[0] if rows is None else rows.numel()
-        l0 = self.shared[0]
-        z1 = self._l1_forward(x16, l0.weight, l0.bias, 0, rows)
+        l0, ln1, l1, ln2 = (self.shared[i] for i in (0, 1, 3, 4))
         heads = (self.move_head, self.bomb_head, self.critic)
-        w1 = self.shared[3].weight.detach().contiguous()
-        wh = torch.cat([h[0].weight.detach() for h in heads]).contiguous()
-        wf = torch.cat([h[2].weight.detach() for h in heads]).contiguous()      # (8, 64)
-        bf = torch.cat([h[2].bias.detach() for h in heads]).contiguous()
-        bh = torch.cat([h[0].bias.detach() for h in heads]).contiguous()
-        f32 = dict(dtype=torch.float32, device=dev)
-        nb = -(-b // 16)
-        # dz2, dhy, dl come chunk-transposed ([chunk][column][row]) and h1,
-        # h2, hy padded to whole chunks, so the weight gradients are batched
-        # products over row chunks with no copies; the padding rows are zero
-        ch = self.GRAD_CHUNK
-        nc = -(-b // ch)
-        bp = nc * ch
-        out = dict(dz1=torch.empty((b, HID), **f32), h1=torch.empty((bp, HID), **f32),
-                   dz2=torch.empty((nc, HID, ch), **f32), h2=torch.empty((bp, HID), **f32),
-                   hy=torch.empty((bp, 3 * HEAD), **f32),
-                   dhy=torch.empty((nc, 3 * HEAD, ch), **f32),
-                   dl=torch.empty((nc, 8, ch), **f32), ln_part=torch.empty((nb, 4, HID), **f32),
-                   stats_part=torch.empty((nb, 5), **f32),
-                   bias_part=torch.empty((nb, 2 * HID + 3 * HEAD + 8), **f32),
-                   dz1_absmax_part=torch.empty((nb, HID), **f32))
-        keep = dict(z1=z1, ln1_w=self.shared[1].weight.detach().contiguous(),
-                    ln1_b=self.shared[1].bias.detach().contiguous(), w1=_kfrag(w1),
-                    w1t=_kfrag(w1.t()), b1=self.shared[3].bias.detach().contiguous(),
-                    ln2_w=self.shared[4].weight.detach().contiguous(),
-                    ln2_b=self.shared[4].bias.detach().contiguous(), wh=_kfrag(wh),
-                    wht=_kfrag(wh.t()), bh=bh, wf=wf, bf=bf,
-                    actions=actions.to(torch.int64).contiguous(),
-                    move_mask=move_mask.to(torch.uint8).contiguous(),
-                    bomb_mask=bomb_mask.to(torch.uint8).contiguous(),
-                    old_logp=old_logp.float().contiguous(), adv=adv.float().contiguous(),
-                    ret=ret.float().contiguous(), old_val=old_val.float().contiguous())
-        a = _capi.PpoArgsC()
+        if [h[2].weight.shape[0] for h in heads] != [5, 2, 1]:
+            raise ValueError("ppo_grads serves heads of 5 moves, 2 bomb actions and the value")
+        z1 = self._l1_forward(x16, l0.weight, l0.bias, 0, rows)
+        a = _capi.PpoStepArgsC()
+        keep = []
+
+        def put(name, t, slot=None):
+            keep.append(t)
+            if slot is None:
+                setattr(a, name, t.data_ptr())
+            else:
+                getattr(a, name)[slot] = t.data_ptr()
+
+        def param(name, p, slot=None):      # the parameter itself and its new gradient
+            put(name, p.detach().float().contiguous(), slot)
+            p.grad = torch.empty(p.shape, dtype=torch.float32, device=dev)
+            put("d" + name, p.grad, slot)
+
+        for name, p in (("ln1_w", ln1.weight), ("ln1_b", ln1.bias), ("w1", l1.weight),
+                        ("b1", l1.bias), ("ln2_w", ln2.weight), ("ln2_b", ln2.bias)):
+            param(name, p)
+        for i, h in enumerate(heads):
+            for name, p in (("wh", h[0].weight), ("bh", h[0].bias), ("wf", h[2].weight),
+                            ("bf", h[2].bias)):
+                param(name, p, i)
         if rows is not None:
             n = x16.shape[0]
             if any(t.shape[0] != n for t in (move_mask, bomb_mask, actions, old_logp, adv, ret,
                                               old_val)):
                 raise ValueError("with rows, every per-row argument must be a whole buffer")
             a.row_index, a.src_rows = rows.data_ptr(), n
-        a.batch = b
+        f32 = dict(dtype=torch.float32, device=dev)
+        dz1, scale, stats = (torch.empty(s, **f32) for s in ((b, HID), (1,), (5,)))
+        l0.bias.grad = torch.empty((HID,), **f32)
+        need = int(self._lib.qqt_ppo_step_workspace_bytes(b))
+        for name, t in (("z1", z1), ("actions", actions.to(torch.int64).contiguous()),
+                        ("move_mask", move_mask.to(torch.uint8).contiguous()),
+                        ("bomb_mask", bomb_mask.to(torch.uint8).contiguous()),
+                        ("old_logp", old_logp.float().contiguous()), ("adv", adv.float().contiguous()),
+                        ("ret", ret.float().contiguous()), ("old_val", old_val.float().contiguous()),
+                        ("dz1", dz1), ("dz_scale", scale), ("stats", stats), ("db0", l0.bias.grad),
+                        ("workspace", torch.empty((need,), dtype=torch.uint8, device=dev))):
+            put(name, t)
+        a.batch, a.workspace_bytes = b, need
         a.clip_eps = cfg.clip_eps
         a.ratio_lo, a.ratio_hi = 1 - cfg.clip_eps, 1 + cfg.clip_eps
         a.value_coef, a.entropy_coef = cfg.value_coef, entropy_coef
-        a.t_chunk = ch
-        if bp > b:
-            for k in ("h1", "h2", "hy"):
-                out[k][b:].zero_()
-            for k in ("dz2", "dhy", "dl"):
-                out[k][-1, :, b - (nc - 1) * ch:].zero_()
-        for k, v in list(keep.items()) + list(out.items()):
-            setattr(a, k, v.data_ptr())
-        _capi.check(self._lib.qqt_ppo_grad(a, _capi.stream_handle(dev)))
-        dz1, dz2, dhy, dl = out["dz1"], out["dz2"], out["dhy"], out["dl"]
-        h1, h2, hy = out["h1"], out["h2"], out["hy"]
-        bias = out["bias_part"].sum(0)            # column sums of dz1 | dz2 | dhy | dl
-        l0.weight.grad = self._l1_weight_grad(x16, dz1, 0, out["dz1_absmax_part"].amax(), rows)
-        l0.bias.grad = bias[:HID].clone()
-        ln = out["ln_part"].sum(0)
-        self.shared[1].weight.grad, self.shared[1].bias.grad = ln[0], ln[1]
-        self.shared[4].weight.grad, self.shared[4].bias.grad = ln[2], ln[3]
-        self.shared[3].weight.grad = torch.bmm(dz2, h1.view(nc, ch, HID)).sum(0)
-        self.shared[3].bias.grad = bias[HID:2 * HID].clone()
-        dwh = torch.bmm(dhy, h2.view(nc, ch, HID)).sum(0)
-        dwf = torch.bmm(dl, hy.view(nc, ch, 3 * HEAD)).sum(0)     # (8, 192): blocks per head
-        dbh = bias[2 * HID:2 * HID + 3 * HEAD]
-        dlb = bias[2 * HID + 3 * HEAD:]
-        rows = 0
-        for i, h in enumerate(heads):
-            h[0].weight.grad = dwh[HEAD * i:HEAD * (i + 1)].contiguous()
-            h[0].bias.grad = dbh[HEAD * i:HEAD * (i + 1)].contiguous()
-            n_out = h[2].weight.shape[0]
-            h[2].weight.grad = dwf[rows:rows + n_out, HEAD * i:HEAD * (i + 1)].contiguous()
-            h[2].bias.grad = dlb[rows:rows + n_out].clone()
-            rows += n_out
-        return out["stats_part"].sum(0) / b
+        _capi.check(self._lib.qqt_ppo_step(a, _capi.stream_handle(dev)))
+        l0.weight.grad = self._l1_weight_grad(x16, dz1, 0, scale=scale, rows=rows)
+        return stats
 
     def evaluate(self, obs, move_mask, bomb_mask, actions, pid: int = 0):
         """(logp, entropy, value) of given actions (train/model.py:247-256)."""

@@ -1,0 +1,112 @@
+"""qqt_ppo_step (the fused PPO minibatch with in-kernel weight gradients)
+against float64 torch from the same first-layer output (needs an MI355X),
+and its argument checks (no GPU needed)."""
+
+import ctypes
+
+import pytest
+import torch
+
+K0 = 14 * 13 * 13
+
+
+def _case(b, seed, dev, outliers):
+    g = torch.Generator().manual_seed(seed)
+    obs = (torch.rand((b, K0), generator=g) < 0.2).half().to(dev)
+    mm = (torch.rand((b, 5), generator=g) < 0.6).to(dev)
+    mm[:, 4] = True
+    bm = torch.ones((b, 2), dtype=torch.bool, device=dev)
+    bm[:, 1] = (torch.rand(b, generator=g) < 0.5).to(dev)
+    act = torch.stack([torch.multinomial(mm.float().cpu(), 1, generator=g)[:, 0],
+                       torch.multinomial(bm.float().cpu(), 1, generator=g)[:, 0]], 1).to(dev)
+    f = lambda s: (s * torch.randn(b, generator=g)).to(dev)  # noqa: E731
+    old_logp, adv, ret, old_val = f(0.3) - 1.5, f(1.0), f(1.0), f(1.0)
+    if outliers:                 # the running scale of the gradients falls in a later tile
+        adv[b // 2], ret[-1] = 3e4, 1e5
+    return obs, mm, bm, act, old_logp, adv, ret, old_val
+
+
+def _float64(net, z1, mm, bm, act, old_logp, adv, ret, old_val, cfg):
+    """Gradients of the minibatch loss above layer 1 (train/ppo.py:408-421)."""
+    w = {k: v.detach().double().requires_grad_(True) for k, v in net.named_parameters()
+         if k != "shared.0.weight"}
+    ln = torch.nn.functional.layer_norm
+    x = z1.double() + (w["shared.0.bias"] - w["shared.0.bias"].detach())
+    x = torch.relu(ln(x, (128,), w["shared.1.weight"], w["shared.1.bias"]))
+    x = x @ w["shared.3.weight"].t() + w["shared.3.bias"]
+    x = torch.relu(ln(x, (128,), w["shared.4.weight"], w["shared.4.bias"]))
+    o = []
+    for h in ("move_head", "bomb_head", "critic"):
+        y = torch.relu(x @ w[f"{h}.0.weight"].t() + w[f"{h}.0.bias"])
+        o.append(y @ w[f"{h}.2.weight"].t() + w[f"{h}.2.bias"])
+    logp, ent = 0.0, 0.0
+    for lg, mask, a in ((o[0], mm, act[:, 0]), (o[1], bm, act[:, 1])):
+        ls = torch.log_softmax(lg.masked_fill(~mask, torch.finfo(torch.float32).min), -1)
+        logp = logp + ls.gather(-1, a[:, None])[:, 0]
+        ent = ent - (ls.exp() * ls).sum(-1)
+    v, e = o[2][:, 0], cfg.clip_eps
+    ratio = (logp - old_logp.double()).exp()
+    pg = -torch.min(ratio * adv, ratio.clamp(1 - e, 1 + e) * adv).mean()
+    vc = old_val + (v - old_val).clamp(-e, e)
+    vf = 0.5 * torch.maximum((v - ret) ** 2, (vc - ret) ** 2).mean()
+    (pg + cfg.value_coef * vf - 0.05 * ent.mean()).backward()
+    return {k: p.grad for k, p in w.items()}, torch.stack([pg, vf, ent.mean()]).detach()
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("outliers", [False, True])
+@pytest.mark.parametrize("b", [1, 31, 32, 33, 100, 8193])
+def test_gradients_against_float64(b, outliers):
+    """Batches around the 32-row tile, one past a whole round of the 256
+    workgroups, and a batch whose gradients span nine orders of magnitude.
+    Bound: float32 products of 128 and 192 terms through four layers are
+    within 3e-6 relative; a hidden unit within rounding of zero may pass or
+    block its ReLU gradient, one row's share of the sum, so 2e-4 beyond a few
+    rows (the outlier row carries its whole sum)."""
+    from qqtsim import HipMlpActorCritic, PPOConfig, reference_init
+
+    dev = torch.device("cuda:0")
+    sd = reference_init(seed=b)
+    for k in sd:
+        if k.endswith("2.weight"):
+            sd[k] = sd[k] + 0.1 * torch.randn(sd[k].shape, generator=torch.Generator().manual_seed(1))
+    net = HipMlpActorCritic(device=dev, state_dict=sd)
+    cfg = PPOConfig()
+    args = _case(b, b, dev, outliers)
+    z1 = net._l1_forward(args[0], net.shared[0].weight, net.shared[0].bias, 0)
+    want, want_st = _float64(net, z1, *args[1:], cfg)
+    st = net.ppo_grads(*args, cfg, 0.05)
+    for k, p in net.named_parameters():
+        if k in want:
+            scale = want[k].norm()
+            err = float((p.grad.double() - want[k]).norm())
+            assert err <= (2e-4 if b > 32 else 3e-6) * float(scale) + 1e-12, (k, err / float(scale))
+    assert float(((st[:3] - want_st) / want_st.abs().clamp_min(1.0)).abs().max()) <= 1e-5
+    dw0 = net.shared[0].weight.grad
+    assert bool(torch.isfinite(dw0).all()) and float(dw0.abs().max()) > 0.0
+
+
+def test_bad_arguments_are_refused():
+    from qqtsim import _capi
+
+    lib = _capi.lib()
+    a = _capi.PpoStepArgsC()
+    assert lib.qqt_ppo_step(ctypes.byref(a), None) == -1
+    assert lib.qqt_last_error() == b"qqt_ppo_step: null argument"
+    assert lib.qqt_ppo_step_workspace_bytes(0) == -1
+    one, many = (lib.qqt_ppo_step_workspace_bytes(n) for n in (1, 1 << 30))
+    assert 0 < one < many < 64 << 20
+    for name, kind in _capi.PpoStepArgsC._fields_:
+        if kind is ctypes.c_void_p:
+            setattr(a, name, 4096)
+        elif kind is ctypes.c_void_p * 3:
+            for i in range(3):
+                getattr(a, name)[i] = 4096
+    a.batch, a.src_rows, a.workspace_bytes = 1, 1, one
+    for field, value, msg in (("batch", 0, b"bad batch"), ("clip_eps", -1.0, b"bad batch"),
+                              ("z1", 4100, b"alignment"), ("workspace_bytes", one - 1, b"too small"),
+                              ("src_rows", 0, b"row_index")):
+        old = getattr(a, field)
+        setattr(a, field, value)
+        assert lib.qqt_ppo_step(ctypes.byref(a), None) == -1 and msg in lib.qqt_last_error(), field
+        setattr(a, field, old)
