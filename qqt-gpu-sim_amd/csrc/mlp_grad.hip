@@ -11,17 +11,24 @@
 // largest magnitude is 2^14) and split into float16 hi + lo, two products per
 // tile, which keeps the result within ~1e-6 relative of a float32 sum.
 //
-// Grid: (column tile of 256 observation columns) x (chunk of the batch).  A
-// workgroup (8 wavefronts) owns a 128 x 256 fp32 output tile for its chunk
-// and walks the chunk 32 rows at a time: each step loads 32 x 256 float16 of
-// the observation and 32 x 128 of dz1 into registers one step ahead, writes
-// them transposed into LDS (the MFMA operands need the batch index
-// contiguous), one barrier per step.  Partial tiles go to a workspace
-// [chunk][128][tiles*256]; a second kernel sums the chunks in a fixed order
+// Grid: (column tile of 512 observation columns) x (chunk of the batch).  A
+// workgroup (8 wavefronts, one per CU) owns a 128 x 512 float32 output tile
+// for its chunk, 64 x 128 per wavefront in registers, and walks the chunk 32
+// rows at a time.  Each step's 32 KB of observation and 16 KB of dz1 are
+// loaded two steps ahead into registers and stored to LDS as they are, row by
+// row (dz1 as hi and lo planes); the MFMA operands, which need the batch index
+// contiguous per lane, are read through the transposing ds_read_b64_tr_b16.
+// One barrier per step.  Partial tiles go to a workspace
+// [chunk][128][tiles*512]; a second kernel sums the chunks in a fixed order
 // (deterministic) and applies the inverse scale.
 //
-// Algorithmic bytes per row: 2 * k0 (observation) + 512 (dz1, read once per
-// column tile: ceil(k0 / 256) times).
+// Bound: HBM, 2 k0 + 512 bytes per row (the observation once; dz1 once per
+// column tile, the repeats from the caches), beside 128 k0 multiply-adds per
+// row in two products.  Tiles of 256 columns (two workgroups per CU) read and
+// split dz1 twice as often, transposed both operands with VALU permutes and
+// had one step of loads in flight: a 180,224-row minibatch of scattered rows
+// took 335 us, now 294; with its rows cached 230, about the rate a library
+// float16 product of 8192^3 reaches on the same card (1.2 PFLOP/s: 180 us).
 
 #include <hip/hip_fp16.h>
 #include <hip/hip_runtime.h>
@@ -32,6 +39,7 @@
 
 #include "qqt_common.h"
 #include "qqt_hip.h"
+#include "qqt_learn.h"
 
 namespace qqt {
 
@@ -43,139 +51,179 @@ typedef _Float16 half8 __attribute__((ext_vector_type(8)));
 typedef float floatx4 __attribute__((ext_vector_type(4)));
 
 constexpr int HID = 128;          // first-layer outputs
-constexpr int NCOL = 256;         // observation columns per workgroup
+constexpr int NCOL = 512;         // observation columns per workgroup
 constexpr int KS = 32;            // batch rows per step (one MFMA K)
-constexpr int XS = KS + 8;        // LDS row stride (halves) of the transposed tiles
+// LDS row strides (halves), 8 banks apart per row: 16-byte stores and the
+// transposing reads (4 rows of 32 bytes per 16 lanes) are conflict-free
+constexpr int XS = NCOL + 16, DS = HID + 16;
 constexpr int NT = 512;           // threads
 constexpr int MAX_CHUNKS = 64;
-constexpr int TARGET_WGS = 512;  // two workgroups (80 KB of LDS each) on each of the 256 CUs
-constexpr int MIN_CHUNK_ROWS = 2048;
+constexpr int TARGET_WGS = 256;   // one workgroup (104 KB of LDS, 256 registers) per CU
+constexpr int MIN_CHUNK_ROWS = 2048;  // in the workspace every caller provides
+constexpr int FINE_CHUNK_ROWS = 512;  // in the preferred workspace
+
+typedef short s4 __attribute__((ext_vector_type(4)));
+typedef __attribute__((address_space(3))) s4 lds_s4;
+typedef uint32_t u32x4 __attribute__((ext_vector_type(4)));
 
 struct __align__(16) Lds {
-  uint16_t xt[2][NCOL][XS];       // observation, [column][row]
-  uint16_t dt[2][2][HID][XS];     // dz1 hi and lo planes, [hidden][row]
+  uint16_t x[2][KS][XS];          // observation rows
+  uint16_t d[2][2][KS][DS];       // dz1 rows, hi and lo planes
 };
 
-__device__ __forceinline__ half8 ld8(const uint16_t* p) {
-  union { uint4 u; half8 h; } c;
-  c.u = *reinterpret_cast<const uint4*>(p);
-  return c.h;
+// Element i of lane (r16, q): row 8q + i, column 16 tile + r16 of an LDS plane
+// with row stride S: lanes 4a..4a+3 of a 16-lane group address row 8q + a
+// (32 bytes) and lane j receives column j of those four rows.
+template <int S>
+__device__ __forceinline__ half8 ld_rows(const uint16_t* plane, int tile, int lane) {
+  const int q = lane >> 4, j = lane & 15;
+  const uint16_t* p = plane + (8 * q + (j >> 2)) * S + 16 * tile + 4 * (j & 3);
+  const s4 a = __builtin_amdgcn_ds_read_tr16_b64_v4i16((lds_s4*)(p));
+  const s4 b = __builtin_amdgcn_ds_read_tr16_b64_v4i16((lds_s4*)(p + 4 * S));
+  return __builtin_bit_cast(half8, __builtin_shufflevector(a, b, 0, 1, 2, 3, 4, 5, 6, 7));
 }
 
-__device__ __forceinline__ uint32_t pack2(float a, float b) {
-  return (uint32_t)__half_as_ushort(__float2half_rn(a)) |
-         ((uint32_t)__half_as_ushort(__float2half_rn(b)) << 16);
-}
-
-__global__ __launch_bounds__(NT) void l1_grad_kernel(const qqt_l1_grad_args a, int chunk_rows,
-                                                     int ws_cols) {
-  __shared__ Lds s;
+// EDGE: the tile reaches past column k0 (or its rows are shorter than a
+// 16-byte chunk): loads go dword by dword, clamped into the row; columns at
+// or past k0 hold repeats that only reach output columns nobody reads.
+template <bool EDGE>
+__device__ __forceinline__ void l1_grad_tile(const qqt_l1_grad_args& a, Lds& s, int tile, int chunk,
+                                             int chunk_rows, int ws_cols) {
   const int t = threadIdx.x;
   const int w = __builtin_amdgcn_readfirstlane(t >> 6), lane = t & 63;
-  const int col0 = blockIdx.x * NCOL;
-  const int r_begin = blockIdx.y * chunk_rows;
+  const int col0 = tile * NCOL;
+  const int r_begin = chunk * chunk_rows;
   const int r_end = min(r_begin + chunk_rows, a.batch);
   const int steps = (r_end - r_begin + KS - 1) / KS;     // >= 1 (chunks are non-empty)
   const float scale = a.dz_scale ? *a.dz_scale : 1.0f;
 
-  // loader roles: observation dword column xd (columns 2xd, 2xd+1) of rows
-  // 8xg..8xg+7; dz1 hidden pair hd (2hd, 2hd+1) of rows 4dg..4dg+3
-  const int xd = t & 127, xg = w >> 1;                    // xg = t >> 7, as a scalar
-  const int hd = t & 63, dg = t >> 6;
-  const bool xcol_ok = col0 + 2 * xd < a.k0;              // k0 is even
-  const uint32_t* const xbase = reinterpret_cast<const uint32_t*>(a.obs);
-  const size_t xstride = (size_t)a.obs_stride / 2;
-
-  uint32_t xr[8];
-  float2 dr[4];
-  auto load = [&](int step) {
+  // loader roles: wavefront w brings rows 4w .. 4w + 3 of the observation,
+  // lane l columns 8l .. 8l + 7; thread t row t / 16 of dz1, hidden 8 (t % 16)
+  // .. + 7.  Rows past the chunk: its last row again, against zero gradients.
+  const int dr = t >> 4, dc = 8 * (t & 15);
+  struct Regs {
+    u32x4 x[4];
+    float d[8];
+  };
+  // Rows of the wavefront in a step: lane l holds the buffer row of row
+  // 4w + l % 4, loaded a step before the observation rows it points at (and
+  // before that step's loads, so waiting for it waits for nothing younger).
+  int64_t at;
+  auto index = [&](int step) {
+    const int r = min(r_begin + KS * step + 4 * w + (lane & 3), r_end - 1);
+    at = a.row_index ? a.row_index[r] : (int64_t)r;
+  };
+  auto load = [&](int step, Regs& g) {
     const int r0 = r_begin + KS * step;
-#pragma unroll
-    for (int i = 0; i < 8; ++i) {
-      const int r = r0 + 8 * xg + i;
-      xr[i] = (r < r_end && xcol_ok) ? xbase[obs_row(a, r) * xstride + (col0 >> 1) + xd] : 0u;
-    }
+    const int64_t row = a.row_index ? min(max(at, (int64_t)0), a.obs_rows - 1) : at;
+    const int lo = (int)row, hi = (int)(row >> 32);
+    index(min(step + 1, steps - 1));
 #pragma unroll
     for (int i = 0; i < 4; ++i) {
-      const int r = r0 + 4 * dg + i;
-      dr[i] = r < r_end ? *reinterpret_cast<const float2*>(a.dz1 + (size_t)r * HID + 2 * hd)
-                        : make_float2(0.0f, 0.0f);
+      const int64_t ri = (int64_t)(((uint64_t)(uint32_t)__builtin_amdgcn_readlane(hi, i) << 32) |
+                                   (uint32_t)__builtin_amdgcn_readlane(lo, i));
+      const uint16_t* const p = a.obs + ri * a.obs_stride;
+      if constexpr (EDGE) {
+#pragma unroll
+        for (int k = 0; k < 4; ++k)
+          g.x[i][k] = reinterpret_cast<const uint32_t*>(p)[min((col0 >> 1) + 4 * lane + k,
+                                                               (a.k0 >> 1) - 1)];
+      } else {
+        __builtin_memcpy(&g.x[i], p + col0 + 8 * lane, 16);      // 4-byte aligned
+      }
     }
+    __builtin_memcpy(g.d, a.dz1 + (size_t)min(r0 + dr, r_end - 1) * HID + dc, 32);
   };
-  auto store = [&](int buf) {
-    uint32_t lo4[4], hi4[4];
+  auto store = [&](const Regs& g, int buf, int step) {
+    const bool live = r_begin + KS * step + dr < r_end;
 #pragma unroll
-    for (int i = 0; i < 4; ++i) {
-      lo4[i] = (xr[2 * i] & 0xFFFFu) | (xr[2 * i + 1] << 16);            // column 2xd
-      hi4[i] = (xr[2 * i] >> 16) | (xr[2 * i + 1] & 0xFFFF0000u);        // column 2xd+1
-    }
-    *reinterpret_cast<uint4*>(&s.xt[buf][2 * xd][8 * xg]) = make_uint4(lo4[0], lo4[1], lo4[2], lo4[3]);
-    *reinterpret_cast<uint4*>(&s.xt[buf][2 * xd + 1][8 * xg]) =
-        make_uint4(hi4[0], hi4[1], hi4[2], hi4[3]);
-    float v0[4], v1[4], l0[4], l1[4];
+    for (int i = 0; i < 4; ++i) *reinterpret_cast<u32x4*>(&s.x[buf][4 * w + i][8 * lane]) = g.x[i];
+    half8 hi, lo;
 #pragma unroll
-    for (int i = 0; i < 4; ++i) {
-      v0[i] = dr[i].x * scale;
-      v1[i] = dr[i].y * scale;
-      l0[i] = v0[i] - __half2float(__float2half_rn(v0[i]));
-      l1[i] = v1[i] - __half2float(__float2half_rn(v1[i]));
+    for (int k = 0; k < 8; ++k) {
+      const float v = live ? g.d[k] * scale : 0.0f;
+      hi[k] = (_Float16)v;
+      lo[k] = (_Float16)(v - (float)hi[k]);
     }
-    *reinterpret_cast<uint2*>(&s.dt[buf][0][2 * hd][4 * dg]) =
-        make_uint2(pack2(v0[0], v0[1]), pack2(v0[2], v0[3]));
-    *reinterpret_cast<uint2*>(&s.dt[buf][0][2 * hd + 1][4 * dg]) =
-        make_uint2(pack2(v1[0], v1[1]), pack2(v1[2], v1[3]));
-    *reinterpret_cast<uint2*>(&s.dt[buf][1][2 * hd][4 * dg]) =
-        make_uint2(pack2(l0[0], l0[1]), pack2(l0[2], l0[3]));
-    *reinterpret_cast<uint2*>(&s.dt[buf][1][2 * hd + 1][4 * dg]) =
-        make_uint2(pack2(l1[0], l1[1]), pack2(l1[2], l1[3]));
+    *reinterpret_cast<half8*>(&s.d[buf][0][dr][dc]) = hi;
+    *reinterpret_cast<half8*>(&s.d[buf][1][dr][dc]) = lo;
   };
 
-  // wavefront w: hidden rows 32(w&3)..+31 (two m tiles), columns 128(w>>2)..+127
-  const int mw = 32 * (w & 3), nw = 128 * (w >> 2);
-  const int r16 = lane & 15, kq = 8 * (lane >> 4);
-  floatx4 acc[2][8];
+  // wavefront w: hidden 64 (w & 1) .. + 63 (four m tiles), columns 128 (w / 2) .. + 127
+  const int mt = 4 * (w & 1), nt = 8 * (w >> 1);
+  const int r16 = lane & 15;
+  floatx4 acc[4][8];
 #pragma unroll
-  for (int i = 0; i < 2; ++i)
+  for (int i = 0; i < 4; ++i)
 #pragma unroll
     for (int j = 0; j < 8; ++j) acc[i][j] = floatx4{0.0f, 0.0f, 0.0f, 0.0f};
-
-  load(0);
-  store(0);
-  __syncthreads();
-  for (int step = 0; step < steps; ++step) {
-    const int buf = step & 1;
-    if (step + 1 < steps) load(step + 1);
-    half8 ah[2], al[2];
+  auto compute = [&](int buf) {
+    half8 ah[4], al[4];
 #pragma unroll
-    for (int i = 0; i < 2; ++i) {
-      ah[i] = ld8(&s.dt[buf][0][mw + 16 * i + r16][kq]);
-      al[i] = ld8(&s.dt[buf][1][mw + 16 * i + r16][kq]);
+    for (int i = 0; i < 4; ++i) {
+      ah[i] = ld_rows<DS>(&s.d[buf][0][0][0], mt + i, lane);
+      al[i] = ld_rows<DS>(&s.d[buf][1][0][0], mt + i, lane);
     }
 #pragma unroll
     for (int j = 0; j < 8; ++j) {
-      const half8 b = ld8(&s.xt[buf][nw + 16 * j + r16][kq]);
+      const half8 b = ld_rows<XS>(&s.x[buf][0][0], nt + j, lane);
 #pragma unroll
-      for (int i = 0; i < 2; ++i) {
-        acc[i][j] = __builtin_amdgcn_mfma_f32_16x16x32_f16(ah[i], b, acc[i][j], 0, 0, 0);
-        acc[i][j] = __builtin_amdgcn_mfma_f32_16x16x32_f16(al[i], b, acc[i][j], 0, 0, 0);
-      }
+      for (int i = 0; i < 4; ++i) acc[i][j] = __builtin_amdgcn_mfma_f32_16x16x32_f16(ah[i], b, acc[i][j], 0, 0, 0);
+#pragma unroll
+      for (int i = 0; i < 4; ++i) acc[i][j] = __builtin_amdgcn_mfma_f32_16x16x32_f16(al[i], b, acc[i][j], 0, 0, 0);
     }
-    if (step + 1 < steps) store(buf ^ 1);
+  };
+
+  // Register ring of two steps in flight beside the LDS double buffer: step i
+  // computes from buffer i & 1, stores step i + 1 to the other and loads step
+  // i + 3 into the slot that freed (steps past the last reload the last).
+  Regs g[2];
+  const int last = steps - 1;
+  index(0);
+  load(0, g[0]);
+  load(min(1, last), g[1]);
+  store(g[0], 0, 0);
+  load(min(2, last), g[0]);
+  __syncthreads();
+  int i = 0;
+  for (; i + 2 <= last; i += 2) {
+#pragma unroll
+    for (int k = 0; k < 2; ++k) {
+      compute(k);
+      store(g[1 - k], 1 - k, i + k + 1);
+      load(min(i + k + 3, last), g[1 - k]);
+      __syncthreads();
+    }
+  }
+  compute(0);
+  if (i < last) {
+    store(g[1], 1, last);
     __syncthreads();
+    compute(1);
   }
 
-  // partial tile -> workspace [chunk][hidden][ws_cols]; lane holds rows
+  // partial tile -> workspace [chunk][hidden][ws_cols]; lane holds hidden rows
   // 4(lane/16)+q of each m tile at column lane%16 of each n tile
-  float* const out = a.workspace + (size_t)blockIdx.y * HID * ws_cols + col0;
+  float* const out = a.workspace + (size_t)chunk * HID * ws_cols + col0;
 #pragma unroll
-  for (int i = 0; i < 2; ++i)
+  for (int i2 = 0; i2 < 4; ++i2)
 #pragma unroll
     for (int j = 0; j < 8; ++j)
 #pragma unroll
-      for (int q = 0; q < 4; ++q) {
-        const int m = mw + 16 * i + 4 * (lane >> 4) + q;
-        out[(size_t)m * ws_cols + nw + 16 * j + r16] = acc[i][j][q];
-      }
+      for (int q = 0; q < 4; ++q)
+        out[(size_t)(16 * (mt + i2) + 4 * (lane >> 4) + q) * ws_cols + 16 * (nt + j) + r16] = acc[i2][j][q];
+}
+
+// (Dealing the column tiles of a chunk to one XCD, so that its L2 serves dz1
+// to all of them, leaves 240 of the 256 CUs at work and measured 308 us
+// against 294; tiles of 256 columns, two workgroups per CU, 317 us.)
+__global__ __launch_bounds__(NT) void l1_grad_kernel(const qqt_l1_grad_args a, int chunk_rows,
+                                                     int ws_cols) {
+  __shared__ Lds s;
+  if ((int)(blockIdx.x + 1) * NCOL <= a.k0)
+    l1_grad_tile<false>(a, s, blockIdx.x, blockIdx.y, chunk_rows, ws_cols);
+  else
+    l1_grad_tile<true>(a, s, blockIdx.x, blockIdx.y, chunk_rows, ws_cols);
 }
 
 // dw0[h][k] = (sum over chunks, in chunk order) / scale, k < k0.
@@ -190,21 +238,25 @@ __global__ __launch_bounds__(256) void l1_grad_reduce(const qqt_l1_grad_args a, 
   a.dw0[i] = sum * inv;
 }
 
-// Chunks of the batch: rows per chunk a multiple of KS, at least
-// MIN_CHUNK_ROWS, and chunks x column tiles at most TARGET_WGS (all
-// workgroups resident at once, evenly two per CU) and MAX_CHUNKS.  (A
-// 180,224-row minibatch of 2366 columns: 51 chunks x 10 tiles = 510
-// workgroups, 374 us; 32 chunks = 320 workgroups left 192 CUs with one
-// workgroup and took 526 us; 64 chunks need a second round, 478 us.)
-__host__ inline void plan(int batch, int k0, int& chunks, int& chunk_rows) {
+// Chunks of the batch: rows per chunk a multiple of KS, at least min_rows, and
+// chunks x column tiles at most TARGET_WGS (all workgroups resident at once,
+// one per CU) and MAX_CHUNKS: a 180,224-row minibatch of 2366 columns makes 51
+// chunks x 5 tiles.
+__host__ inline void plan(int batch, int k0, int min_rows, int& chunks, int& chunk_rows) {
   const int tiles = (k0 + NCOL - 1) / NCOL;
-  chunks = (batch + MIN_CHUNK_ROWS - 1) / MIN_CHUNK_ROWS;
+  chunks = (batch + min_rows - 1) / min_rows;
   if (chunks > TARGET_WGS / tiles) chunks = TARGET_WGS / tiles;
   if (chunks > MAX_CHUNKS) chunks = MAX_CHUNKS;
   if (chunks < 1) chunks = 1;
   chunk_rows = (batch + chunks - 1) / chunks;
   chunk_rows = (chunk_rows + KS - 1) / KS * KS;
   chunks = (batch + chunk_rows - 1) / chunk_rows;
+}
+
+__host__ inline int64_t plan_floats(int batch, int k0, int min_rows) {
+  int chunks, rows;
+  plan(batch, k0, min_rows, chunks, rows);
+  return (int64_t)chunks * HID * ((k0 + NCOL - 1) / NCOL) * NCOL;
 }
 
 }  // namespace l1g
@@ -253,10 +305,13 @@ extern "C" {
 int64_t qqt_l1_grad_workspace_floats(int32_t batch, int32_t k0) {
   using namespace qqt::l1g;
   if (batch <= 0 || k0 <= 0) return -1;
-  int chunks, rows;
-  plan(batch, k0, chunks, rows);
-  const int tiles = (k0 + NCOL - 1) / NCOL;
-  return (int64_t)chunks * HID * tiles * NCOL;
+  return plan_floats(batch, k0, MIN_CHUNK_ROWS);
+}
+
+int64_t qqt_l1_grad_preferred_floats(int32_t batch, int32_t k0) {
+  using namespace qqt::l1g;
+  if (batch <= 0 || k0 <= 0) return -1;
+  return plan_floats(batch, k0, FINE_CHUNK_ROWS);
 }
 
 namespace {
@@ -286,8 +341,15 @@ int l1_grad_check(const qqt_l1_grad_args* a, const char* who) {
 int l1_grad_launch(const qqt_l1_grad_args& a, hipStream_t st) {
   using namespace qqt;
   using namespace qqt::l1g;
+  // Finer chunks where the workspace holds them: chunks of 2048 rows leave an
+  // 8192-row batch on 20 workgroups (136 us with its reduction; 35 us in 16
+  // chunks of 512).  Below 512 rows the partial tiles (1.3 MB per chunk out
+  // and back) cost what the shorter walk saves.
   int chunks, rows;
-  plan(a.batch, a.k0, chunks, rows);
+  plan(a.batch, a.k0,
+       a.workspace_floats >= plan_floats(a.batch, a.k0, FINE_CHUNK_ROWS) ? FINE_CHUNK_ROWS
+                                                                         : MIN_CHUNK_ROWS,
+       chunks, rows);
   const int tiles = (a.k0 + NCOL - 1) / NCOL;
   const int ws_cols = tiles * NCOL;
   QQT_LAUNCH(QQT_KERNEL_L1GRAD, l1_grad_kernel, dim3(tiles, chunks), dim3(NT), st, a, rows,
@@ -337,8 +399,8 @@ int qqt_l1_grad_noalloc(const qqt_l1_grad_args* a, void* stream) {
   if (!ptr) return QQT_E_LAUNCH;
   qqt_l1_grad_args b = *a;          // the caller's workspace fields are ignored
   b.workspace = ptr;
-  b.workspace_floats = (int64_t)l1g::MAX_CHUNKS * l1g::HID * QQT_L1_GRAD_NOALLOC_MAX_K0;
-  if (b.workspace_floats < qqt_l1_grad_workspace_floats(b.batch, b.k0)) {
+  b.workspace_floats = qqt_l1_grad_workspace_floats(b.batch, b.k0);
+  if (b.workspace_floats > (int64_t)l1g::MAX_CHUNKS * l1g::HID * QQT_L1_GRAD_NOALLOC_MAX_K0) {
     snprintf(g_err, sizeof(g_err), "qqt_l1_grad_noalloc: plan exceeds the static scratch");
     return QQT_E_ARG;
   }

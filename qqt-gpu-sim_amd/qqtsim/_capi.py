@@ -189,6 +189,8 @@ def lib():
         L.qqt_l1_grad_workspace_floats.argtypes = [_i32, _i32]
         L.qqt_ppo_grad.restype = ctypes.c_int
         L.qqt_ppo_grad.argtypes = [ctypes.POINTER(PpoArgsC), _vp]
+        L.qqt_l1_grad_preferred_floats.restype = ctypes.c_int64
+        L.qqt_l1_grad_preferred_floats.argtypes = [_i32, _i32]
         L.qqt_ppo_step.restype = ctypes.c_int
         L.qqt_ppo_step.argtypes = [ctypes.POINTER(PpoStepArgsC), _vp]
         L.qqt_ppo_step_workspace_bytes.restype = ctypes.c_int64

@@ -176,7 +176,7 @@ class HipMlpActorCritic(nn.Module):
         when the caller has it."""
         a = _capi.L1GradArgsC()
         b = self._rows_args(a, x16, rows)
-        need = int(self._lib.qqt_l1_grad_workspace_floats(b, self.k0))
+        need = int(self._lib.qqt_l1_grad_preferred_floats(b, self.k0))
         if self._ws is None or self._ws.numel() < need:
             self._ws = torch.empty(need, dtype=torch.float32, device=x16.device)
         if scale is None:
@@ -184,7 +184,7 @@ class HipMlpActorCritic(nn.Module):
             scale = torch.exp2(torch.clamp(14.0 - torch.ceil(torch.log2(amax)), -100.0, 100.0))
         dw0p = torch.empty((HID, self.k0), dtype=torch.float32, device=x16.device)
         a.batch, a.k0, a.obs_stride = b, self.k0, x16.stride(0)
-        a.workspace_floats = self._ws.numel()
+        a.workspace_floats = need            # the plan follows it, not the buffer's history
         a.obs, a.dz1, a.dz_scale = x16.data_ptr(), dz1.data_ptr(), scale.data_ptr()
         a.workspace, a.dw0 = self._ws.data_ptr(), dw0p.data_ptr()
         _capi.check(self._lib.qqt_l1_grad(a, _capi.stream_handle(x16.device)))
