@@ -64,6 +64,28 @@ int qqt_ppo_step(const qqt_ppo_step_args* args, void* stream);
  * exactly this many in workspace_floats to get the finer plan. */
 int64_t qqt_l1_grad_preferred_floats(int32_t batch, int32_t k0);
 
+/* The recurrent part of the lstm learner over whole sequences (train/ppo.py:
+ * 463-490): gate order i, f, g, o, hidden width 128, the state entering frame
+ * 0 zero, the state after frame t multiplied by keep[t].  All arrays are
+ * contiguous float32; T = steps, M = rows (envs). */
+typedef struct qqt_lstm_seq_args {
+  int32_t steps, rows;
+  int32_t window;             /* backward: no gradient passes into frame t from frame t + 1's
+                                 state when t + 1 is a multiple of it (0: never cut) */
+  int32_t pad;
+  const float* w_hh;          /* [512][128], 16-byte aligned */
+  const float* keep;          /* [T][M] */
+  const float* zx;            /* [T][M][512] W_ih x + both biases (forward) */
+  float* h;                   /* [T][M][128] out: h before keep (forward) */
+  float* c;                   /* [T][M][128] c before keep: out of forward, in of backward */
+  float* gates;               /* [T][M][512] gate values: out of forward, in of backward */
+  const float* dh;            /* [T][M][128] gradient of h (backward) */
+  float* dz;                  /* [T][M][512] out: gradient of z = zx + W_hh h (backward) */
+} qqt_lstm_seq_args;
+
+int qqt_lstm_seq_forward(const qqt_lstm_seq_args* args, void* stream);
+int qqt_lstm_seq_backward(const qqt_lstm_seq_args* args, void* stream);
+
 #ifdef __cplusplus
 }
 #endif

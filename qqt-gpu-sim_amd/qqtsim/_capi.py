@@ -160,6 +160,11 @@ class GaeArgsC(ctypes.Structure):
         (n, _vp) for n in ("rew", "val", "done", "last_val", "adv", "ret")]
 
 
+class LstmSeqArgsC(ctypes.Structure):
+    _fields_ = [("steps", _i32), ("rows", _i32), ("window", _i32), ("pad", _i32)] + [
+        (n, _vp) for n in ("w_hh", "keep", "zx", "h", "c", "gates", "dh", "dz")]
+
+
 _LIB = None
 
 
@@ -204,6 +209,9 @@ def lib():
         L.qqt_gather_rows.argtypes = [ctypes.POINTER(GatherArgsC), _vp]
         L.qqt_lstm_act.restype = ctypes.c_int
         L.qqt_lstm_act.argtypes = [ctypes.POINTER(LstmArgsC), _vp]
+        for fn in (L.qqt_lstm_seq_forward, L.qqt_lstm_seq_backward):
+            fn.restype = ctypes.c_int
+            fn.argtypes = [ctypes.POINTER(LstmSeqArgsC), _vp]
         L.qqt_timing_arm.restype = ctypes.c_int
         L.qqt_timing_arm.argtypes = [_i32]
         L.qqt_timing_collect.restype = ctypes.c_int

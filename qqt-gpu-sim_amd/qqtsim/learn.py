@@ -100,6 +100,25 @@ class _Linear(torch.autograd.Function):
         return dy @ w, _weight_grad(dy, x), dy.sum(0)
 
 
+class _InputProduct(_Linear):
+    """The same product for the recurrence's inputs, summed over quarters of
+    the reduction: one sum over all 256 inputs leaves an error in the gates
+    that is larger than everything the recurrence adds (hidden outputs of 32
+    frames x 256 envs against float64, mean of eight inputs: 1.37e-7 relative
+    with one sum, 1.05e-7 with quarters, 1.06e-7 through nn.LSTM's own
+    kernels)."""
+
+    @staticmethod
+    def forward(ctx, x, w, b):
+        ctx.save_for_backward(x, w)
+        step = -(-x.shape[1] // 4)
+        parts = [(x[:, k:k + step], w[:, k:k + step].t()) for k in range(0, x.shape[1], step)]
+        out = torch.addmm(b, *parts[0])
+        for p in parts[1:]:
+            out.addmm_(*p)
+        return out
+
+
 def _lin(mod: nn.Linear, x):
     return _Linear.apply(x, mod.weight, mod.bias)
 
@@ -470,6 +489,84 @@ def _masked_logp_entropy(ml, bl, mm, bm, act):
     return logp, ent
 
 
+class _Recurrence(torch.autograd.Function):
+    """(T, m, 128) hidden outputs of the recurrence z = zx + h W_hh^T over T
+    frames from the zero state, the state multiplied by keep[t] after frame t
+    and detached every `window` frames (0 = never): one launch forward, one
+    backward (`qqt_lstm_seq_*`).  W_hh's gradient is one product over all
+    frames after the first."""
+
+    @staticmethod
+    def forward(ctx, zx, w_hh, keep, window):
+        steps, m = keep.shape
+        new = lambda width: torch.empty((steps, m, width), dtype=torch.float32,  # noqa: E731
+                                        device=zx.device)
+        h, c, gates = new(HID), new(HID), new(4 * HID)
+        a = _capi.LstmSeqArgsC()
+        a.steps, a.rows, a.window = steps, m, window
+        a.w_hh, a.keep, a.zx = w_hh.data_ptr(), keep.data_ptr(), zx.data_ptr()
+        a.h, a.c, a.gates = h.data_ptr(), c.data_ptr(), gates.data_ptr()
+        _capi.check(_capi.lib().qqt_lstm_seq_forward(a, _capi.stream_handle(zx.device)))
+        ctx.save_for_backward(w_hh, keep, h, c, gates)
+        ctx.window = window
+        return h
+
+    @staticmethod
+    @torch.autograd.function.once_differentiable
+    def backward(ctx, dh):
+        w_hh, keep, h, c, gates = ctx.saved_tensors
+        w_hh, keep, h, c, gates, dh = (t.contiguous() for t in (w_hh, keep, h, c, gates, dh))
+        dz = torch.empty_like(gates)
+        a = _capi.LstmSeqArgsC()
+        a.steps, a.rows, a.window = *keep.shape, ctx.window
+        a.w_hh, a.keep, a.c, a.gates = (t.data_ptr() for t in (w_hh, keep, c, gates))
+        a.dh, a.dz = dh.data_ptr(), dz.data_ptr()
+        _capi.check(_capi.lib().qqt_lstm_seq_backward(a, _capi.stream_handle(dh.device)))
+        dw = None
+        if ctx.needs_input_grad[1]:
+            if keep.shape[0] > 1:
+                before = (h[:-1] * keep[:-1].unsqueeze(-1)).view(-1, HID)
+                dw = _weight_grad(dz[1:].view(-1, 4 * HID), before, chunk=1024)
+            else:
+                dw = torch.zeros_like(w_hh)
+        return dz if ctx.needs_input_grad[0] else None, dw, None, None
+
+
+def _sequence_kernels_serve(lstm, x) -> bool:
+    """Whether `_Recurrence` stands for the module's own call frame by frame:
+    a plain float32 nn.LSTM of this network's shape on the GPU, with nothing
+    hooked into its call or its parameters' use."""
+    if type(lstm) is not nn.LSTM or not x.is_cuda or x.dtype != torch.float32:
+        return False
+    if (lstm.num_layers, lstm.hidden_size, lstm.bidirectional, lstm.proj_size, lstm.bias,
+            lstm.batch_first) != (1, HID, False, 0, True, True):
+        return False
+    if "forward" in vars(lstm) or any(getattr(lstm, k, None) for k in (
+            "_forward_hooks", "_forward_pre_hooks", "_backward_hooks", "_backward_pre_hooks")):
+        return False
+    mod = torch.nn.modules.module
+    if any(getattr(mod, k, None) for k in ("_global_forward_hooks", "_global_forward_pre_hooks",
+                                           "_global_backward_hooks",
+                                           "_global_backward_pre_hooks")):
+        return False
+    if torch.is_autocast_enabled() or torch.compiler.is_compiling():
+        return False
+    w = (lstm.weight_ih_l0, lstm.weight_hh_l0, lstm.bias_ih_l0, lstm.bias_hh_l0)
+    return all(p.dtype == torch.float32 and p.device == x.device for p in w)
+
+
+def _sequence_outputs(lstm, fused, keep, window: int):
+    """(T, m, 128) outputs of the LSTM over the fused features (T, m, 256):
+    the input products of all frames together, then the recurrence."""
+    steps, m, width = fused.shape
+    zx = _InputProduct.apply(fused.reshape(steps * m, width), lstm.weight_ih_l0,
+                       lstm.bias_ih_l0 + lstm.bias_hh_l0)
+    w_hh = lstm.weight_hh_l0.contiguous()
+    if w_hh.data_ptr() % 16:
+        w_hh = w_hh.clone()
+    return _Recurrence.apply(zx.view(steps, m, -1).contiguous(), w_hh, keep.contiguous(), window)
+
+
 def _lstm_update(learner, opt, buf, last_val, cfg: PPOConfig, entropy_coef: float) -> dict:
     """PPO over an lstm rollout buffer (train/ppo.py:440-537).  Minibatches
     are sets of envs with their whole T-step sequences: per epoch one
@@ -478,7 +575,9 @@ def _lstm_update(learner, opt, buf, last_val, cfg: PPOConfig, entropy_coef: floa
     per-frame features of all T x N_sub frames go through `extract_fused`
     at once; the LSTM then runs over t = 0..T-1 from the zero state, its
     state multiplied by (1 - done[t]) after each frame and detached every
-    `bptt_window` frames (0 = never); the heads and the masked log-probs
+    `bptt_window` frames (0 = never), as one forward and one backward launch
+    where `_sequence_kernels_serve` says so (frame by frame through the module
+    it is about 1,500 launches per minibatch of 32 frames); the heads and the masked log-probs
     run on all frames together.  The clipped surrogate, the clipped value
     loss and the entropy bonus use the GAE advantages normalised over the
     whole buffer (unbiased std + 1e-8); then gradient clipping and one
@@ -503,15 +602,19 @@ def _lstm_update(learner, opt, buf, last_val, cfg: PPOConfig, entropy_coef: floa
             frames = [x[:, envs].reshape(steps * m, *x.shape[2:])
                       for x in (buf.local, buf.rel, buf.glob)]
             fused = learner.extract_fused(*frames).view(steps, m, -1)
-            k = keep[:, envs].view(steps, 1, m, 1)
-            state, outs = None, []
-            for t in range(steps):
-                if window > 0 and t % window == 0 and state is not None:
-                    state = (state[0].detach(), state[1].detach())
-                out, state = learner.lstm(fused[t].unsqueeze(1), state)
-                outs.append(out.squeeze(1))
-                state = (state[0] * k[t], state[1] * k[t])
-            ml, bl, value = learner.heads(torch.stack(outs))
+            if steps > 0 and _sequence_kernels_serve(learner.lstm, fused):
+                hidden = _sequence_outputs(learner.lstm, fused, keep[:, envs], max(0, window))
+            else:
+                k = keep[:, envs].view(steps, 1, m, 1)
+                state, outs = None, []
+                for t in range(steps):
+                    if window > 0 and t % window == 0 and state is not None:
+                        state = (state[0].detach(), state[1].detach())
+                    out, state = learner.lstm(fused[t].unsqueeze(1), state)
+                    outs.append(out.squeeze(1))
+                    state = (state[0] * k[t], state[1] * k[t])
+                hidden = torch.stack(outs)
+            ml, bl, value = learner.heads(hidden)
             logp, ent = _masked_logp_entropy(ml, bl, mm[:, envs], bm[:, envs], act[:, envs])
             a, r, ov, ol = adv[:, envs], ret[:, envs], old_val[:, envs], old_logp[:, envs]
             ratio = torch.exp(logp - ol)

@@ -1,0 +1,99 @@
+"""qqt_lstm_seq_forward / _backward (the lstm learner's recurrence over whole
+sequences) against the frame-by-frame recurrence in float64 torch."""
+
+from __future__ import annotations
+
+import ctypes
+
+import pytest
+import torch
+
+HID = 128
+
+
+def _frame_by_frame(x, lstm, keep, window):
+    """The update's recurrence (train/ppo.py:463-490) from the module's
+    weights in float64: outputs (T, m, 128)."""
+    h = c = torch.zeros((x.shape[1], HID), dtype=x.dtype, device=x.device)
+    outs = []
+    for t in range(x.shape[0]):
+        if window > 0 and t % window == 0:
+            h, c = h.detach(), c.detach()
+        z = (x[t] @ lstm.weight_ih_l0.t() + lstm.bias_ih_l0 + h @ lstm.weight_hh_l0.t()
+             + lstm.bias_hh_l0)
+        i, f, g, o = z.chunk(4, -1)
+        c = torch.sigmoid(f) * c + torch.sigmoid(i) * torch.tanh(g)
+        h = torch.sigmoid(o) * torch.tanh(c)
+        outs.append(h)
+        h, c = h * keep[t][:, None], c * keep[t][:, None]
+    return torch.stack(outs)
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("steps,m,window", [(1, 1, 0), (2, 15, 0), (7, 16, 3), (33, 17, 8),
+                                            (8, 31, 1), (32, 256, 0), (128, 37, 16)])
+def test_sequence_kernels_match_the_frame_by_frame_recurrence(steps, m, window):
+    from qqtsim.learn import _sequence_kernels_serve, _sequence_outputs
+
+    torch.manual_seed(steps * 1000 + m)
+    lstm = torch.nn.LSTM(256, HID, batch_first=True).cuda()
+    x = torch.randn(steps, m, 256, device="cuda").relu().requires_grad_(True)
+    keep = (torch.rand(steps, m, device="cuda") > 0.1).float()
+    dy = torch.randn(steps, m, HID, device="cuda")
+    assert _sequence_kernels_serve(lstm, x)
+    out = _sequence_outputs(lstm, x, keep, window)
+    out.backward(dy)
+    ref = torch.nn.LSTM(256, HID, batch_first=True).cuda().double()
+    ref.load_state_dict({k: v.double() for k, v in lstm.state_dict().items()})
+    x64 = x.detach().double().requires_grad_(True)
+    want = _frame_by_frame(x64, ref, keep.double(), window)
+    want.backward(dy.double())
+
+    def rel(a, b):
+        return float((a.double() - b).norm() / b.norm().clamp_min(1e-30))
+
+    # float32 sums of up to 512 terms and steps m rows: a few times
+    # sqrt(512) 2^-24 = 1.3e-6 per product, carried through the frames
+    assert rel(out, want) < 2e-6
+    assert rel(x.grad, x64.grad) < 5e-6
+    for (k, p), (_, q) in zip(lstm.named_parameters(), ref.named_parameters()):
+        assert rel(p.grad, q.grad) < 5e-6, k
+
+
+def test_only_a_plain_float32_lstm_on_the_gpu_is_served():
+    from qqtsim.learn import _sequence_kernels_serve
+
+    class Lstm(torch.nn.LSTM):
+        pass
+
+    x = torch.zeros(2, 3, 256)
+    assert not _sequence_kernels_serve(torch.nn.LSTM(256, HID, batch_first=True), x)
+    assert not _sequence_kernels_serve(Lstm(256, HID, batch_first=True), x)
+    if torch.cuda.is_available():
+        x = x.cuda()
+        lstm = torch.nn.LSTM(256, HID, batch_first=True).cuda()
+        assert _sequence_kernels_serve(lstm, x)
+        hook = lstm.register_forward_hook(lambda *a: None)
+        assert not _sequence_kernels_serve(lstm, x)
+        hook.remove()
+        assert not _sequence_kernels_serve(lstm.double(), x)
+
+
+def test_bad_arguments_are_refused():
+    from qqtsim import _capi
+
+    lib = _capi.lib()
+    for fn, own in ((lib.qqt_lstm_seq_forward, ("zx", "h")), (lib.qqt_lstm_seq_backward, ("dh", "dz"))):
+        def args():
+            a = _capi.LstmSeqArgsC(steps=4, rows=3)
+            for k in ("w_hh", "keep", "c", "gates") + own:
+                setattr(a, k, 4096)
+            return a
+        for k in ("w_hh", "keep", "c", "gates") + own:
+            a = args()
+            setattr(a, k, None)
+            assert fn(ctypes.byref(a), None) == -1 and b"null argument" in lib.qqt_last_error(), k
+        for k, v in (("steps", 0), ("rows", -1), ("window", -1), ("w_hh", 4100)):
+            a = args()
+            setattr(a, k, v)
+            assert fn(ctypes.byref(a), None) == -1 and b"bad steps" in lib.qqt_last_error(), k
