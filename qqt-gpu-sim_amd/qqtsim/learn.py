@@ -270,7 +270,9 @@ class HipMlpActorCritic(nn.Module):
                 getattr(a, name)[slot] = t.data_ptr()
 
         def param(name, p, slot=None):      # the parameter itself and its new gradient
-            put(name, p.detach().float().contiguous(), slot)
+            t = p.detach().float().contiguous()
+            # a parameter that is a view into a flat buffer may lie at any element
+            put(name, t.clone() if t.data_ptr() % 16 else t, slot)
             p.grad = torch.empty(p.shape, dtype=torch.float32, device=dev)
             put("d" + name, p.grad, slot)
 

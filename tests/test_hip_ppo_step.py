@@ -86,6 +86,30 @@ def test_gradients_against_float64(b, outliers):
     assert bool(torch.isfinite(dw0).all()) and float(dw0.abs().max()) > 0.0
 
 
+@pytest.mark.gpu
+def test_parameters_that_view_a_flat_buffer():
+    """Parameters at any element of one flat buffer (not 16-byte aligned) are
+    served, with the gradients of the same values in tensors of their own."""
+    from qqtsim import HipMlpActorCritic, PPOConfig, reference_init
+
+    dev = torch.device("cuda:0")
+    sd = reference_init(seed=3)
+    args = _case(33, 3, dev, False)
+    own, flat = (HipMlpActorCritic(device=dev, state_dict=sd) for _ in range(2))
+    buf = torch.zeros(1 + sum(p.numel() + 1 for p in flat.parameters()), device=dev)
+    at = 1
+    for p in flat.parameters():
+        view = buf[at:at + p.numel()].view(p.shape)
+        view.copy_(p.detach())
+        p.data = view
+        at += p.numel() + 1
+    assert flat.shared[3].weight.data_ptr() % 16
+    for net in (own, flat):
+        net.ppo_grads(*args, PPOConfig(), 0.05)
+    for (k, p), (_, q) in zip(own.named_parameters(), flat.named_parameters()):
+        assert torch.equal(p.grad, q.grad), k
+
+
 def test_bad_arguments_are_refused():
     from qqtsim import _capi
 
