@@ -64,6 +64,18 @@ int qqt_ppo_step(const qqt_ppo_step_args* args, void* stream);
  * exactly this many in workspace_floats to get the finer plan. */
 int64_t qqt_l1_grad_preferred_floats(int32_t batch, int32_t k0);
 
+/* qqt_l1_grad for an observation whose columns are a permutation of the
+ * weight's: column k of the product is written to column cols[k] of dw0
+ * (cols: [k0] on the device, every value of [0, k0) once). */
+int qqt_l1_grad_columns(const qqt_l1_grad_args* args, const int64_t* cols, void* stream);
+
+/* The first layer's weight (w: [128][k0] float32, contiguous) as the float16
+ * fragments of qqt_mlp_act's w0, its columns taken in the order cols ([k0] on
+ * the device).  out: 128 * 64 * kblocks halves, 16-byte aligned, kblocks the
+ * 64-column blocks that hold k0. */
+int qqt_w0_pack(const float* w, const int64_t* cols, int32_t k0, int32_t kblocks, void* out,
+                void* stream);
+
 /* The recurrent part of the lstm learner over whole sequences (train/ppo.py:
  * 463-490): gate order i, f, g, o, hidden width 128, the state entering frame
  * 0 zero, the state after frame t multiplied by keep[t].  All arrays are

@@ -226,16 +226,53 @@ __global__ __launch_bounds__(NT) void l1_grad_kernel(const qqt_l1_grad_args a, i
     l1_grad_tile<true>(a, s, blockIdx.x, blockIdx.y, chunk_rows, ws_cols);
 }
 
-// dw0[h][k] = (sum over chunks, in chunk order) / scale, k < k0.
+// dw0[h][cols ? cols[k] : k] = (sum over chunks, in chunk order) / scale,
+// k < k0.  A column index outside [0, k0) is clamped into it.  Bound: HBM and
+// the Infinity Cache (51 partials of 1.3 MB for a 180,224-row minibatch); eight
+// loads in flight per thread, added in chunk order.
 __global__ __launch_bounds__(256) void l1_grad_reduce(const qqt_l1_grad_args a, int chunks,
-                                                      int ws_cols) {
+                                                      int ws_cols, const int64_t* cols) {
   const int i = blockIdx.x * 256 + threadIdx.x;
   if (i >= HID * a.k0) return;
   const int h = i / a.k0, k = i % a.k0;
   const float inv = a.dz_scale ? 1.0f / *a.dz_scale : 1.0f;   // power of two: exact
+  const size_t pitch = (size_t)HID * ws_cols;
+  const float* p = a.workspace + (size_t)h * ws_cols + k;
+  const int64_t col = cols ? min(max(cols[k], (int64_t)0), (int64_t)a.k0 - 1) : (int64_t)k;
   float sum = 0.0f;
-  for (int c = 0; c < chunks; ++c) sum += a.workspace[((size_t)c * HID + h) * ws_cols + k];
-  a.dw0[i] = sum * inv;
+  int c = 0;
+  for (; c + 8 <= chunks; c += 8, p += 8 * pitch) {
+    float v[8];
+#pragma unroll
+    for (int j = 0; j < 8; ++j) v[j] = p[j * pitch];
+#pragma unroll
+    for (int j = 0; j < 8; ++j) sum += v[j];
+  }
+  for (; c < chunks; ++c, p += pitch) sum += *p;
+  a.dw0[(size_t)h * a.k0 + col] = sum * inv;
+}
+
+// The first layer's weight as the float16 MFMA B fragments the forward reads,
+// [tile][kblock][lane 16 q + r][16]: value i is row 16 tile + r, column
+// cols[64 kblock + 16 q + i], zero from k0 on.  A thread writes 16 bytes; a
+// launch moves 1.8 MB (1.2 read, 0.6 written) and is latency.  In its place
+// were an index, a fill, two copies and a conversion; with the column order of
+// dW0 (another index launch) folded into l1_grad_reduce, the gradients of an
+// 8192-row minibatch went 192 -> 159 us and of 180,224 rows 895 -> 866 us.
+__global__ __launch_bounds__(256) void w0_pack_kernel(const float* w, const int64_t* cols, int k0,
+                                                      int kblocks, uint16_t* out) {
+  const int i = blockIdx.x * 256 + threadIdx.x;           // 8 halves each
+  if (i >= HID / 16 * kblocks * 128) return;
+  const int lane = (i >> 1) & 63, kb = (i >> 7) % kblocks, tile = (i >> 7) / kblocks;
+  const int k = 64 * kb + 16 * (lane >> 4) + 8 * (i & 1);
+  const float* const row = w + (size_t)(16 * tile + (lane & 15)) * k0;
+  half8 v;
+#pragma unroll
+  for (int j = 0; j < 8; ++j) {
+    const int64_t col = k + j < k0 ? min(max(cols[k + j], (int64_t)0), (int64_t)k0 - 1) : 0;
+    v[j] = k + j < k0 ? (_Float16)row[col] : (_Float16)0.0f;
+  }
+  *reinterpret_cast<half8*>(out + 8 * (size_t)i) = v;
 }
 
 // Chunks of the batch: rows per chunk a multiple of KS, at least min_rows, and
@@ -336,9 +373,22 @@ int l1_grad_check(const qqt_l1_grad_args* a, const char* who) {
   return QQT_OK;
 }
 
+int l1_grad_workspace_check(const qqt_l1_grad_args& a, const char* who) {
+  using namespace qqt;
+  if (!a.workspace) {
+    snprintf(g_err, sizeof(g_err), "%s: null workspace", who);
+    return QQT_E_ARG;
+  }
+  if (a.workspace_floats < qqt_l1_grad_workspace_floats(a.batch, a.k0)) {
+    snprintf(g_err, sizeof(g_err), "%s: workspace too small", who);
+    return QQT_E_ARG;
+  }
+  return QQT_OK;
+}
+
 // Both launches over a checked argument block whose workspace holds the
 // plan's partials.
-int l1_grad_launch(const qqt_l1_grad_args& a, hipStream_t st) {
+int l1_grad_launch(const qqt_l1_grad_args& a, hipStream_t st, const int64_t* cols = nullptr) {
   using namespace qqt;
   using namespace qqt::l1g;
   // Finer chunks where the workspace holds them: chunks of 2048 rows leave an
@@ -358,7 +408,7 @@ int l1_grad_launch(const qqt_l1_grad_args& a, hipStream_t st) {
   if (err == hipSuccess) {
     const int n = HID * a.k0;
     QQT_LAUNCH(QQT_KERNEL_L1GRAD, l1_grad_reduce, dim3((n + 255) / 256), dim3(256), st, a,
-               chunks, ws_cols);
+               chunks, ws_cols, cols);
     err = hipGetLastError();
   }
   if (err != hipSuccess) {
@@ -374,15 +424,44 @@ int qqt_l1_grad(const qqt_l1_grad_args* a, void* stream) {
   using namespace qqt;
   g_err[0] = 0;
   if (const int rc = l1_grad_check(a, "qqt_l1_grad")) return rc;
-  if (!a->workspace) {
-    snprintf(g_err, sizeof(g_err), "qqt_l1_grad: null workspace");
-    return QQT_E_ARG;
-  }
-  if (a->workspace_floats < qqt_l1_grad_workspace_floats(a->batch, a->k0)) {
-    snprintf(g_err, sizeof(g_err), "qqt_l1_grad: workspace too small");
-    return QQT_E_ARG;
-  }
+  if (const int rc = l1_grad_workspace_check(*a, "qqt_l1_grad")) return rc;
   return l1_grad_launch(*a, (hipStream_t)stream);
+}
+
+int qqt_l1_grad_columns(const qqt_l1_grad_args* a, const int64_t* cols, void* stream) {
+  using namespace qqt;
+  g_err[0] = 0;
+  if (const int rc = l1_grad_check(a, "qqt_l1_grad_columns")) return rc;
+  if (const int rc = l1_grad_workspace_check(*a, "qqt_l1_grad_columns")) return rc;
+  if (!cols || (((uintptr_t)cols) & 7)) {
+    snprintf(g_err, sizeof(g_err), "qqt_l1_grad_columns: cols must be an 8-byte aligned device array");
+    return QQT_E_ARG;
+  }
+  return l1_grad_launch(*a, (hipStream_t)stream, cols);
+}
+
+int qqt_w0_pack(const float* w, const int64_t* cols, int32_t k0, int32_t kblocks, void* out,
+                void* stream) {
+  using namespace qqt;
+  using namespace qqt::l1g;
+  g_err[0] = 0;
+  if (!w || !cols || !out) {
+    snprintf(g_err, sizeof(g_err), "qqt_w0_pack: null argument");
+    return QQT_E_ARG;
+  }
+  if (k0 <= 0 || kblocks != (k0 - 1) / 64 + 1 || kblocks > (1 << 20) || (((uintptr_t)w) & 3) ||
+      (((uintptr_t)cols) & 7) || (((uintptr_t)out) & 15)) {
+    snprintf(g_err, sizeof(g_err), "qqt_w0_pack: bad k0, kblocks or alignment");
+    return QQT_E_ARG;
+  }
+  hipLaunchKernelGGL(w0_pack_kernel, dim3(HID / 16 * kblocks * 128 / 256), dim3(256), 0,
+                     (hipStream_t)stream, w, cols, k0, kblocks, static_cast<uint16_t*>(out));
+  const hipError_t err = hipGetLastError();
+  if (err != hipSuccess) {
+    snprintf(g_err, sizeof(g_err), "w0 pack launch failed: %s", hipGetErrorString(err));
+    return QQT_E_LAUNCH;
+  }
+  return QQT_OK;
 }
 
 int qqt_l1_grad_noalloc(const qqt_l1_grad_args* a, void* stream) {

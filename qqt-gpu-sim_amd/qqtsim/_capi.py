@@ -196,6 +196,10 @@ def lib():
         L.qqt_ppo_grad.argtypes = [ctypes.POINTER(PpoArgsC), _vp]
         L.qqt_l1_grad_preferred_floats.restype = ctypes.c_int64
         L.qqt_l1_grad_preferred_floats.argtypes = [_i32, _i32]
+        L.qqt_l1_grad_columns.restype = ctypes.c_int
+        L.qqt_l1_grad_columns.argtypes = [ctypes.POINTER(L1GradArgsC), _vp, _vp]
+        L.qqt_w0_pack.restype = ctypes.c_int
+        L.qqt_w0_pack.argtypes = [_vp, _vp, _i32, _i32, _vp, _vp]
         L.qqt_ppo_step.restype = ctypes.c_int
         L.qqt_ppo_step.argtypes = [ctypes.POINTER(PpoStepArgsC), _vp]
         L.qqt_ppo_step_workspace_bytes.restype = ctypes.c_int64

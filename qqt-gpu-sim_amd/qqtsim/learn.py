@@ -40,15 +40,17 @@ from .policy import (HEAD, HID, KBLOCK, _layer_tree, column_permutation, default
 from .ppo import compute_gae
 
 
-def _w0_fragments(w: torch.Tensor, kpad: int) -> torch.Tensor:
-    """(128, k) float weight on the device -> float16 B fragments
-    [tile][kblock][lane][16] (the layout of qqtsim.policy._frag)."""
+def _w0_fragments(w: torch.Tensor, cols: torch.Tensor) -> torch.Tensor:
+    """(128, k) weight on the device, its columns in the order `cols` ->
+    float16 B fragments [tile][kblock][lane][16] (the layout of
+    qqtsim.policy._frag), one launch."""
+    w = w.detach().float().contiguous()
     n, k = w.shape
-    out = torch.zeros((n, kpad), dtype=torch.float32, device=w.device)
-    out[:, :k] = w
-    kb = kpad // KBLOCK
-    f = out.view(n // 16, 16, kb, 4, 16).permute(0, 2, 3, 1, 4).contiguous()
-    return f.half().reshape(-1)
+    kb = -(-k // KBLOCK)
+    out = torch.empty(n * kb * KBLOCK, dtype=torch.float16, device=w.device)
+    _capi.check(_capi.lib().qqt_w0_pack(w.data_ptr(), cols.data_ptr(), k, kb, out.data_ptr(),
+                                        _capi.stream_handle(w.device)))
+    return out
 
 
 class _FirstLayer(torch.autograd.Function):
@@ -148,9 +150,8 @@ class HipMlpActorCritic(nn.Module):
                              else reference_init(obs_shape, n_moves, n_bomb))
         self.to(dev)
         self._lib = _capi.lib()
-        perms = [column_permutation(pid, n_players, c, h * w) for pid in range(n_players)]
-        self._perm = [p.to(dev) for p in perms]
-        self._inv = [torch.argsort(p).to(dev) for p in perms]
+        self._perm = [column_permutation(pid, n_players, c, h * w).to(dev)
+                      for pid in range(n_players)]
         # the first-layer launch reads the later layers' buffers in its
         # prologue; zero stand-ins of the packed sizes
         packed = pack_mlp(default_init(obs_shape, n_moves, n_bomb), n_players, obs_shape)
@@ -177,7 +178,7 @@ class HipMlpActorCritic(nn.Module):
         a = _capi.MlpArgsC()
         b = self._rows_args(a, x16, rows)
         z1 = torch.empty((b, HID), dtype=torch.float32, device=x16.device)
-        frag = _w0_fragments(w0.detach()[:, self._perm[pid]].float(), self.kpad)
+        frag = _w0_fragments(w0, self._perm[pid])
         bias = b0.detach().float().contiguous()
         a.batch, a.npid, a.pid0, a.sample = b, 1, 0, 0
         a.k0, a.kblocks0, a.obs_stride = self.k0, self.kpad // KBLOCK, x16.stride(0)
@@ -201,13 +202,14 @@ class HipMlpActorCritic(nn.Module):
         if scale is None:
             amax = dz1.abs().amax().clamp_min(1e-30)
             scale = torch.exp2(torch.clamp(14.0 - torch.ceil(torch.log2(amax)), -100.0, 100.0))
-        dw0p = torch.empty((HID, self.k0), dtype=torch.float32, device=x16.device)
+        dw0 = torch.empty((HID, self.k0), dtype=torch.float32, device=x16.device)
         a.batch, a.k0, a.obs_stride = b, self.k0, x16.stride(0)
         a.workspace_floats = need            # the plan follows it, not the buffer's history
         a.obs, a.dz1, a.dz_scale = x16.data_ptr(), dz1.data_ptr(), scale.data_ptr()
-        a.workspace, a.dw0 = self._ws.data_ptr(), dw0p.data_ptr()
-        _capi.check(self._lib.qqt_l1_grad(a, _capi.stream_handle(x16.device)))
-        return dw0p[:, self._inv[pid]]
+        a.workspace, a.dw0 = self._ws.data_ptr(), dw0.data_ptr()
+        _capi.check(self._lib.qqt_l1_grad_columns(a, self._perm[pid].data_ptr(),
+                                                  _capi.stream_handle(x16.device)))
+        return dw0
 
     # ------------------------------------------------------------ API
     def forward(self, obs, pid: int = 0):
@@ -244,9 +246,9 @@ class HipMlpActorCritic(nn.Module):
         player 0's view) written into every parameter's `.grad`, as
         `loss.backward()` through `evaluate` would leave them; returns the
         five statistics (pg, vf, ent, kl, clipfrac) as a device tensor.
-        Three calls: the first layer's forward, `qqt_ppo_step` (the loss, the
-        backward above the first layer and every gradient there) and
-        `qqt_l1_grad`.  With `rows` (int64 indices), every per-row argument (obs,
+        Four calls: the first layer's weight fragments and forward,
+        `qqt_ppo_step` (the loss, the backward above the first layer and every
+        gradient there) and `qqt_l1_grad_columns`.  With `rows` (int64 indices), every per-row argument (obs,
         masks, actions, old log-probs, advantages, returns, old values) is a
         whole buffer and the minibatch is its rows `rows`, which the kernels
         read in place."""
