@@ -1014,8 +1014,8 @@ def main_ppo(args, torch, dev):
         "value": samples / el, "unit": "samples/s", "n_gpus": 1, "steps": reps,
         "warmup": 1, "ms_per_step": el * 1e3, "higher_is_better": True, "scaling": "weak",
         "vs_baseline": None,
-        "dtype": "f16 MFMA first layer (f32 accumulate) / f32 fused loss + backward / f32 torch "
-                 "weight-gradient products and Adam",
+        "dtype": "f16 MFMA first layer (f32 accumulate) / f16 hi/lo pair MFMA fused loss + backward "
+                 "+ weight gradients (f32 accumulate) / f32 torch Adam",
         "data": "synthetic: a buffer collected by the kernels from template maps, acted by "
                 "the learner's weights (the reference ActorCritic's orthogonal init)",
         "config": {"workload": "PPO update over a 5632 x 128 rollout buffer "
@@ -1031,7 +1031,7 @@ def main_ppo(args, torch, dev):
                                                 "bytes_per_row": L1G_BYTES_PER_ROW},
                     "first-layer forward (per minibatch)": {
                         "us": round(fwd_ms * 1e3, 3), "obs_gbs": round(fwd_gbs, 3)},
-                    "ppo_grad_kernel (per minibatch)": {"us": round(ppo_ms * 1e3, 3)}},
+                    "ppo_step_kernel (per minibatch)": {"us": round(ppo_ms * 1e3, 3)}},
         "torch_gpu_baseline": None if el_ref is None else {
             "value": samples / el_ref, "unit": "samples/s", "ms_per_update": el_ref * 1e3,
             "speedup": round(el_ref / el, 3), "update_stats": ref_stats,
