@@ -260,9 +260,12 @@ class HipMlpActorCritic(nn.Module):
         heads = (self.move_head, self.bomb_head, self.critic)
         if [h[2].weight.shape[0] for h in heads] != [5, 2, 1]:
             raise ValueError("ppo_grads serves heads of 5 moves, 2 bomb actions and the value")
+        if rows is not None and any(t.shape[0] != x16.shape[0] for t in (
+                move_mask, bomb_mask, actions, old_logp, adv, ret, old_val)):
+            raise ValueError("with rows, every per-row argument must be a whole buffer")
         z1 = self._l1_forward(x16, l0.weight, l0.bias, 0, rows)
         a = _capi.PpoStepArgsC()
-        keep = []
+        keep, grads = [], []
 
         def put(name, t, slot=None):
             keep.append(t)
@@ -275,8 +278,8 @@ class HipMlpActorCritic(nn.Module):
             t = p.detach().float().contiguous()
             # a parameter that is a view into a flat buffer may lie at any element
             put(name, t.clone() if t.data_ptr() % 16 else t, slot)
-            p.grad = torch.empty(p.shape, dtype=torch.float32, device=dev)
-            put("d" + name, p.grad, slot)
+            grads.append((p, torch.empty(p.shape, dtype=torch.float32, device=dev)))
+            put("d" + name, grads[-1][1], slot)
 
         for name, p in (("ln1_w", ln1.weight), ("ln1_b", ln1.bias), ("w1", l1.weight),
                         ("b1", l1.bias), ("ln2_w", ln2.weight), ("ln2_b", ln2.bias)):
@@ -286,21 +289,16 @@ class HipMlpActorCritic(nn.Module):
                             ("bf", h[2].bias)):
                 param(name, p, i)
         if rows is not None:
-            n = x16.shape[0]
-            if any(t.shape[0] != n for t in (move_mask, bomb_mask, actions, old_logp, adv, ret,
-                                              old_val)):
-                raise ValueError("with rows, every per-row argument must be a whole buffer")
-            a.row_index, a.src_rows = rows.data_ptr(), n
+            a.row_index, a.src_rows = rows.data_ptr(), x16.shape[0]
         f32 = dict(dtype=torch.float32, device=dev)
-        dz1, scale, stats = (torch.empty(s, **f32) for s in ((b, HID), (1,), (5,)))
-        l0.bias.grad = torch.empty((HID,), **f32)
+        dz1, scale, stats, db0 = (torch.empty(s, **f32) for s in ((b, HID), (1,), (5,), (HID,)))
         need = int(self._lib.qqt_ppo_step_workspace_bytes(b))
         for name, t in (("z1", z1), ("actions", actions.to(torch.int64).contiguous()),
                         ("move_mask", move_mask.to(torch.uint8).contiguous()),
                         ("bomb_mask", bomb_mask.to(torch.uint8).contiguous()),
                         ("old_logp", old_logp.float().contiguous()), ("adv", adv.float().contiguous()),
                         ("ret", ret.float().contiguous()), ("old_val", old_val.float().contiguous()),
-                        ("dz1", dz1), ("dz_scale", scale), ("stats", stats), ("db0", l0.bias.grad),
+                        ("dz1", dz1), ("dz_scale", scale), ("stats", stats), ("db0", db0),
                         ("workspace", torch.empty((need,), dtype=torch.uint8, device=dev))):
             put(name, t)
         a.batch, a.workspace_bytes = b, need
@@ -308,7 +306,9 @@ class HipMlpActorCritic(nn.Module):
         a.ratio_lo, a.ratio_hi = 1 - cfg.clip_eps, 1 + cfg.clip_eps
         a.value_coef, a.entropy_coef = cfg.value_coef, entropy_coef
         _capi.check(self._lib.qqt_ppo_step(a, _capi.stream_handle(dev)))
-        l0.weight.grad = self._l1_weight_grad(x16, dz1, 0, scale=scale, rows=rows)
+        grads += [(l0.bias, db0), (l0.weight, self._l1_weight_grad(x16, dz1, 0, scale=scale, rows=rows))]
+        for p, g in grads:      # only now: a call that is refused leaves every `.grad` as it was
+            p.grad = g
         return stats
 
     def evaluate(self, obs, move_mask, bomb_mask, actions, pid: int = 0):

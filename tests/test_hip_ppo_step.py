@@ -110,6 +110,26 @@ def test_parameters_that_view_a_flat_buffer():
         assert torch.equal(p.grad, q.grad), k
 
 
+@pytest.mark.gpu
+def test_a_refused_call_leaves_the_gradients_alone():
+    from qqtsim import HipMlpActorCritic, PPOConfig, reference_init
+
+    dev = torch.device("cuda:0")
+    net = HipMlpActorCritic(device=dev, state_dict=reference_init(seed=4))
+    args = list(_case(40, 4, dev, False))
+    rows = torch.arange(33, device=dev)
+    for fill in (None, 3.0):
+        for p in net.parameters():
+            p.grad = None if fill is None else torch.full_like(p, fill)
+        had = [p.grad for p in net.parameters()]
+        with pytest.raises(ValueError, match="whole buffer"):
+            net.ppo_grads(*args[:-1], args[-1][:33], PPOConfig(), 0.05, rows=rows)
+        with pytest.raises(ValueError, match="clip"):
+            net.ppo_grads(*args, PPOConfig(clip_eps=-1.0), 0.05, rows=rows)
+        assert all(p.grad is g for p, g in zip(net.parameters(), had))
+        assert fill is None or all(bool((g == fill).all()) for g in had)
+
+
 def test_bad_arguments_are_refused():
     from qqtsim import _capi
 
