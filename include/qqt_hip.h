@@ -330,8 +330,10 @@ int qqt_gae(const qqt_gae_args* args, void* stream);
  * float16 MFMA with float32 accumulation; dz1 is multiplied by *dz_scale
  * (a power of two chosen by the caller so that max|dz1| * scale <= 2^14;
  * NULL = 1) before its float16 hi/lo split and the result is divided by it.
- * Deterministic: fixed batch chunks summed in chunk order.  The caller
- * provides the workspace (qqt_l1_grad_workspace_floats floats). */
+ * Deterministic: batch chunks, fixed by batch and k0, summed in a fixed
+ * order.  The caller provides the workspace (at least
+ * qqt_l1_grad_workspace_floats floats; a larger one can be faster and does
+ * not change the result). */
 typedef struct qqt_l1_grad_args {
   int32_t batch;              /* rows B */
   int32_t k0;                 /* observation width C*H*W (even) */
@@ -357,7 +359,7 @@ int qqt_l1_grad(const qqt_l1_grad_args* args, void* stream);
  * floats (80 MiB, one per GPU, held until the process ends); `workspace`
  * and `workspace_floats` are ignored.  Any batch size; k0 at most
  * QQT_L1_GRAD_NOALLOC_MAX_K0 (larger is QQT_E_ARG).  The result equals
- * qqt_l1_grad's bit for bit (same plan, same kernels).  The call allocates
+ * qqt_l1_grad's bit for bit, whatever workspace that has.  The call allocates
  * nothing: its first call on a device looks up the array's address there.
  * Every element of the array that a call reads, the same call wrote first;
  * calls that overlap on one GPU (different streams) race on the array. */

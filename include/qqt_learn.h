@@ -58,10 +58,11 @@ int64_t qqt_ppo_step_workspace_bytes(int32_t batch);
 
 int qqt_ppo_step(const qqt_ppo_step_args* args, void* stream);
 
-/* Workspace (floats) at which qqt_l1_grad cuts a small batch into chunks of
- * 512 rows instead of 2048, so that more workgroups share it (>=
- * qqt_l1_grad_workspace_floats; the sums then run in another order).  Pass
- * exactly this many in workspace_floats to get the finer plan. */
+/* Workspace (floats; at least qqt_l1_grad_workspace_floats) that holds the
+ * partials of every chunk of 512 rows or more, so that each chunk of a small
+ * batch gets its own workgroups; in a smaller one they walk up to four chunks
+ * each.  The result is the same, bit for bit, in any workspace that
+ * qqt_l1_grad accepts. */
 int64_t qqt_l1_grad_preferred_floats(int32_t batch, int32_t k0);
 
 /* qqt_l1_grad for an observation whose columns are a permutation of the

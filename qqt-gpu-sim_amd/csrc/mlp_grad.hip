@@ -11,7 +11,8 @@
 // largest magnitude is 2^14) and split into float16 hi + lo, two products per
 // tile, which keeps the result within ~1e-6 relative of a float32 sum.
 //
-// Grid: (column tile of 512 observation columns) x (chunk of the batch).  A
+// Grid: (column tile of 512 observation columns) x (chunk of the batch); tiles of
+// 128 columns where the workspace has slots for groups of chunks only (Plan).  A
 // workgroup (8 wavefronts, one per CU) owns a 128 x 512 float32 output tile
 // for its chunk, 64 x 128 per wavefront in registers, and walks the chunk 32
 // rows at a time.  Each step's 32 KB of observation and 16 KB of dz1 are
@@ -19,7 +20,7 @@
 // row (dz1 as hi and lo planes); the MFMA operands, which need the batch index
 // contiguous per lane, are read through the transposing ds_read_b64_tr_b16.
 // One barrier per step.  Partial tiles go to a workspace
-// [chunk][128][tiles*512]; a second kernel sums the chunks in a fixed order
+// [slot][128][tiles * width]; a second kernel sums the slots in a fixed order
 // (deterministic) and applies the inverse scale.
 //
 // Bound: HBM, 2 k0 + 512 bytes per row (the observation once; dz1 once per
@@ -51,23 +52,30 @@ typedef _Float16 half8 __attribute__((ext_vector_type(8)));
 typedef float floatx4 __attribute__((ext_vector_type(4)));
 
 constexpr int HID = 128;          // first-layer outputs
-constexpr int NCOL = 512;         // observation columns per workgroup
+constexpr int NCOL = 512;         // observation columns per workgroup ...
+constexpr int NARROW = 128;       // ... and where its slot takes several chunks
 constexpr int KS = 32;            // batch rows per step (one MFMA K)
-// LDS row strides (halves), 8 banks apart per row: 16-byte stores and the
-// transposing reads (4 rows of 32 bytes per 16 lanes) are conflict-free
-constexpr int XS = NCOL + 16, DS = HID + 16;
+// LDS row strides (halves; NC + 16 for the observation), 8 banks apart per row:
+// 16-byte stores and the transposing reads (4 rows of 32 bytes per 16 lanes)
+// are conflict-free
+constexpr int DS = HID + 16;
 constexpr int NT = 512;           // threads
 constexpr int MAX_CHUNKS = 64;
 constexpr int TARGET_WGS = 256;   // one workgroup (104 KB of LDS, 256 registers) per CU
-constexpr int MIN_CHUNK_ROWS = 2048;  // in the workspace every caller provides
-constexpr int FINE_CHUNK_ROWS = 512;  // in the preferred workspace
+constexpr int CHUNK_ROWS = 512;   // least rows of a chunk
+constexpr int SLOT_ROWS = 2048;   // ... of a slot of the workspace every caller provides
 
 typedef short s4 __attribute__((ext_vector_type(4)));
 typedef __attribute__((address_space(3))) s4 lds_s4;
 typedef uint32_t u32x4 __attribute__((ext_vector_type(4)));
 
+__device__ __forceinline__ floatx4 mfma(half8 a, half8 b, floatx4 c) {
+  return __builtin_amdgcn_mfma_f32_16x16x32_f16(a, b, c, 0, 0, 0);
+}
+
+template <int NC>
 struct __align__(16) Lds {
-  uint16_t x[2][KS][XS];          // observation rows
+  uint16_t x[2][KS][NC + 16];     // observation rows
   uint16_t d[2][2][KS][DS];       // dz1 rows, hi and lo planes
 };
 
@@ -83,26 +91,38 @@ __device__ __forceinline__ half8 ld_rows(const uint16_t* plane, int tile, int la
   return __builtin_bit_cast(half8, __builtin_shufflevector(a, b, 0, 1, 2, 3, 4, 5, 6, 7));
 }
 
+// Accumulators of a wavefront: four m tiles x JT n tiles.
+template <int NC>
+struct Tile {
+  static constexpr int JT = NC / 64;
+  floatx4 v[4][JT];
+};
+
+// One chunk's product for a tile of NC columns, from zero.
 // EDGE: the tile reaches past column k0 (or its rows are shorter than a
 // 16-byte chunk): loads go dword by dword, clamped into the row; columns at
 // or past k0 hold repeats that only reach output columns nobody reads.
-template <bool EDGE>
-__device__ __forceinline__ void l1_grad_tile(const qqt_l1_grad_args& a, Lds& s, int tile, int chunk,
-                                             int chunk_rows, int ws_cols) {
+template <int NC, bool EDGE>
+__device__ __forceinline__ void l1_grad_chunk(const qqt_l1_grad_args& a, Lds<NC>& s, int tile,
+                                              int chunk, int chunk_rows, Tile<NC>& acc) {
+  constexpr int XS = NC + 16, JT = Tile<NC>::JT;
+  constexpr int LPR = NC / 8;             // lanes of an observation row (16 bytes each)
+  constexpr int RPL = 64 / LPR, NL = 4 / RPL;    // rows per load, loads per step
   const int t = threadIdx.x;
   const int w = __builtin_amdgcn_readfirstlane(t >> 6), lane = t & 63;
-  const int col0 = tile * NCOL;
+  const int col0 = tile * NC;
   const int r_begin = chunk * chunk_rows;
   const int r_end = min(r_begin + chunk_rows, a.batch);
   const int steps = (r_end - r_begin + KS - 1) / KS;     // >= 1 (chunks are non-empty)
   const float scale = a.dz_scale ? *a.dz_scale : 1.0f;
 
   // loader roles: wavefront w brings rows 4w .. 4w + 3 of the observation,
-  // lane l columns 8l .. 8l + 7; thread t row t / 16 of dz1, hidden 8 (t % 16)
-  // .. + 7.  Rows past the chunk: its last row again, against zero gradients.
+  // lane l columns 8 (l % LPR) .. + 7 of row l / LPR of each load; thread t row
+  // t / 16 of dz1, hidden 8 (t % 16) .. + 7.  Rows past the chunk: its last row
+  // again, against zero gradients.
   const int dr = t >> 4, dc = 8 * (t & 15);
   struct Regs {
-    u32x4 x[4];
+    u32x4 x[NL];
     float d[8];
   };
   // Rows of the wavefront in a step: lane l holds the buffer row of row
@@ -119,17 +139,24 @@ __device__ __forceinline__ void l1_grad_tile(const qqt_l1_grad_args& a, Lds& s, 
     const int lo = (int)row, hi = (int)(row >> 32);
     index(min(step + 1, steps - 1));
 #pragma unroll
-    for (int i = 0; i < 4; ++i) {
-      const int64_t ri = (int64_t)(((uint64_t)(uint32_t)__builtin_amdgcn_readlane(hi, i) << 32) |
-                                   (uint32_t)__builtin_amdgcn_readlane(lo, i));
+    for (int i = 0; i < NL; ++i) {
+      uint32_t rl, rh;
+      if constexpr (RPL == 1) {
+        rl = __builtin_amdgcn_readlane(lo, i);
+        rh = __builtin_amdgcn_readlane(hi, i);
+      } else {
+        rl = __shfl(lo, RPL * i + lane / LPR, 64);
+        rh = __shfl(hi, RPL * i + lane / LPR, 64);
+      }
+      const int64_t ri = (int64_t)(((uint64_t)rh << 32) | rl);
       const uint16_t* const p = a.obs + ri * a.obs_stride;
+      const int c = 8 * (lane % LPR);
       if constexpr (EDGE) {
 #pragma unroll
         for (int k = 0; k < 4; ++k)
-          g.x[i][k] = reinterpret_cast<const uint32_t*>(p)[min((col0 >> 1) + 4 * lane + k,
-                                                               (a.k0 >> 1) - 1)];
+          g.x[i][k] = reinterpret_cast<const uint32_t*>(p)[min(((col0 + c) >> 1) + k, (a.k0 >> 1) - 1)];
       } else {
-        __builtin_memcpy(&g.x[i], p + col0 + 8 * lane, 16);      // 4-byte aligned
+        __builtin_memcpy(&g.x[i], p + col0 + c, 16);             // 4-byte aligned
       }
     }
     __builtin_memcpy(g.d, a.dz1 + (size_t)min(r0 + dr, r_end - 1) * HID + dc, 32);
@@ -137,7 +164,8 @@ __device__ __forceinline__ void l1_grad_tile(const qqt_l1_grad_args& a, Lds& s, 
   auto store = [&](const Regs& g, int buf, int step) {
     const bool live = r_begin + KS * step + dr < r_end;
 #pragma unroll
-    for (int i = 0; i < 4; ++i) *reinterpret_cast<u32x4*>(&s.x[buf][4 * w + i][8 * lane]) = g.x[i];
+    for (int i = 0; i < NL; ++i)
+      *reinterpret_cast<u32x4*>(&s.x[buf][4 * w + RPL * i + lane / LPR][8 * (lane % LPR)]) = g.x[i];
     half8 hi, lo;
 #pragma unroll
     for (int k = 0; k < 8; ++k) {
@@ -149,28 +177,41 @@ __device__ __forceinline__ void l1_grad_tile(const qqt_l1_grad_args& a, Lds& s, 
     *reinterpret_cast<half8*>(&s.d[buf][1][dr][dc]) = lo;
   };
 
-  // wavefront w: hidden 64 (w & 1) .. + 63 (four m tiles), columns 128 (w / 2) .. + 127
-  const int mt = 4 * (w & 1), nt = 8 * (w >> 1);
-  const int r16 = lane & 15;
-  floatx4 acc[4][8];
+  // wavefront w: hidden 64 (w & 1) .. + 63 (four m tiles), column quarter w / 2
+  const int mt = 4 * (w & 1), nt = JT * (w >> 1);
 #pragma unroll
   for (int i = 0; i < 4; ++i)
 #pragma unroll
-    for (int j = 0; j < 8; ++j) acc[i][j] = floatx4{0.0f, 0.0f, 0.0f, 0.0f};
+    for (int j = 0; j < JT; ++j) acc.v[i][j] = floatx4{0.0f, 0.0f, 0.0f, 0.0f};
   auto compute = [&](int buf) {
-    half8 ah[4], al[4];
+    if constexpr (NC == NARROW) {       // few n tiles: hold those, pass the m tiles through
+      half8 b[JT];
 #pragma unroll
-    for (int i = 0; i < 4; ++i) {
-      ah[i] = ld_rows<DS>(&s.d[buf][0][0][0], mt + i, lane);
-      al[i] = ld_rows<DS>(&s.d[buf][1][0][0], mt + i, lane);
-    }
+      for (int j = 0; j < JT; ++j) b[j] = ld_rows<XS>(&s.x[buf][0][0], nt + j, lane);
 #pragma unroll
-    for (int j = 0; j < 8; ++j) {
-      const half8 b = ld_rows<XS>(&s.x[buf][0][0], nt + j, lane);
+      for (int i = 0; i < 4; ++i) {
+        const half8 ah = ld_rows<DS>(&s.d[buf][0][0][0], mt + i, lane);
+        const half8 al = ld_rows<DS>(&s.d[buf][1][0][0], mt + i, lane);
 #pragma unroll
-      for (int i = 0; i < 4; ++i) acc[i][j] = __builtin_amdgcn_mfma_f32_16x16x32_f16(ah[i], b, acc[i][j], 0, 0, 0);
+        for (int j = 0; j < JT; ++j) acc.v[i][j] = mfma(ah, b[j], acc.v[i][j]);
 #pragma unroll
-      for (int i = 0; i < 4; ++i) acc[i][j] = __builtin_amdgcn_mfma_f32_16x16x32_f16(al[i], b, acc[i][j], 0, 0, 0);
+        for (int j = 0; j < JT; ++j) acc.v[i][j] = mfma(al, b[j], acc.v[i][j]);
+      }
+    } else {
+      half8 ah[4], al[4];
+#pragma unroll
+      for (int i = 0; i < 4; ++i) {
+        ah[i] = ld_rows<DS>(&s.d[buf][0][0][0], mt + i, lane);
+        al[i] = ld_rows<DS>(&s.d[buf][1][0][0], mt + i, lane);
+      }
+#pragma unroll
+      for (int j = 0; j < JT; ++j) {
+        const half8 b = ld_rows<XS>(&s.x[buf][0][0], nt + j, lane);
+#pragma unroll
+        for (int i = 0; i < 4; ++i) acc.v[i][j] = mfma(ah[i], b, acc.v[i][j]);
+#pragma unroll
+        for (int i = 0; i < 4; ++i) acc.v[i][j] = mfma(al[i], b, acc.v[i][j]);
+      }
     }
   };
 
@@ -201,36 +242,66 @@ __device__ __forceinline__ void l1_grad_tile(const qqt_l1_grad_args& a, Lds& s, 
     __syncthreads();
     compute(1);
   }
-
-  // partial tile -> workspace [chunk][hidden][ws_cols]; lane holds hidden rows
-  // 4(lane/16)+q of each m tile at column lane%16 of each n tile
-  float* const out = a.workspace + (size_t)chunk * HID * ws_cols + col0;
-#pragma unroll
-  for (int i2 = 0; i2 < 4; ++i2)
-#pragma unroll
-    for (int j = 0; j < 8; ++j)
-#pragma unroll
-      for (int q = 0; q < 4; ++q)
-        out[(size_t)(16 * (mt + i2) + 4 * (lane >> 4) + q) * ws_cols + 16 * (nt + j) + r16] = acc[i2][j][q];
 }
 
+// Column tile blockIdx.x of slot blockIdx.y -> workspace [slot][hidden][ws_cols].
+// A slot takes one chunk in the wide tile; in the narrow one up to `per_slot`
+// consecutive chunks, their products added in order in registers.
 // (Dealing the column tiles of a chunk to one XCD, so that its L2 serves dz1
 // to all of them, leaves 240 of the 256 CUs at work and measured 308 us
-// against 294; tiles of 256 columns, two workgroups per CU, 317 us.)
-__global__ __launch_bounds__(NT) void l1_grad_kernel(const qqt_l1_grad_args a, int chunk_rows,
-                                                     int ws_cols) {
-  __shared__ Lds s;
-  if ((int)(blockIdx.x + 1) * NCOL <= a.k0)
-    l1_grad_tile<false>(a, s, blockIdx.x, blockIdx.y, chunk_rows, ws_cols);
-  else
-    l1_grad_tile<true>(a, s, blockIdx.x, blockIdx.y, chunk_rows, ws_cols);
+// against 294; tiles of 256 columns, two workgroups per CU, 317 us.  Adding a
+// slot's chunks in the workspace instead, which the wide tile would need, took
+// 232 us for 8,192 rows in four slots.)  The narrow tile is held to 128 registers
+// (13 go to scratch): two workgroups per CU take 45,056 rows in 17 slots in
+// 115 us, one (156 registers) in 134.
+template <int NC, bool EDGE>
+__device__ __forceinline__ void l1_grad_slot(const qqt_l1_grad_args& a, Lds<NC>& s, int chunks,
+                                             int chunk_rows, int ws_cols, int per_slot) {
+  constexpr int JT = Tile<NC>::JT;
+  Tile<NC> sum;
+  if constexpr (NC == NARROW) {
+    const int first = blockIdx.y * per_slot, end = min(first + per_slot, chunks);
+#pragma unroll 1
+    for (int c = first; c < end; ++c) {
+      Tile<NC> acc;
+      l1_grad_chunk<NC, EDGE>(a, s, blockIdx.x, c, chunk_rows, acc);
+#pragma unroll
+      for (int i = 0; i < 4; ++i)
+#pragma unroll
+        for (int j = 0; j < JT; ++j) sum.v[i][j] = c == first ? acc.v[i][j] : sum.v[i][j] + acc.v[i][j];
+      __syncthreads();                  // every wavefront is done with this chunk's LDS
+    }
+  } else {
+    l1_grad_chunk<NC, EDGE>(a, s, blockIdx.x, blockIdx.y, chunk_rows, sum);
+  }
+  // lane holds hidden rows 4(lane/16)+q of each m tile at column lane%16 of each n tile
+  const int w = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), lane = threadIdx.x & 63;
+  const int mt = 4 * (w & 1), nt = JT * (w >> 1);
+  float* const out = a.workspace + (size_t)blockIdx.y * HID * ws_cols + blockIdx.x * NC;
+#pragma unroll
+  for (int i = 0; i < 4; ++i)
+#pragma unroll
+    for (int j = 0; j < JT; ++j)
+#pragma unroll
+      for (int q = 0; q < 4; ++q)
+        out[(size_t)(16 * (mt + i) + 4 * (lane >> 4) + q) * ws_cols + 16 * (nt + j) + (lane & 15)] = sum.v[i][j][q];
 }
 
-// dw0[h][cols ? cols[k] : k] = (sum over chunks, in chunk order) / scale,
-// k < k0.  A column index outside [0, k0) is clamped into it.  Bound: HBM and
-// the Infinity Cache (51 partials of 1.3 MB for a 180,224-row minibatch); eight
-// loads in flight per thread, added in chunk order.
-__global__ __launch_bounds__(256) void l1_grad_reduce(const qqt_l1_grad_args a, int chunks,
+template <int NC>
+__global__ __launch_bounds__(NT, NC == NARROW ? 4 : 2) void l1_grad_kernel(
+    const qqt_l1_grad_args a, int chunks, int chunk_rows, int ws_cols, int per_slot) {
+  __shared__ Lds<NC> s;
+  if ((int)(blockIdx.x + 1) * NC <= a.k0)
+    l1_grad_slot<NC, false>(a, s, chunks, chunk_rows, ws_cols, per_slot);
+  else
+    l1_grad_slot<NC, true>(a, s, chunks, chunk_rows, ws_cols, per_slot);
+}
+
+// dw0[h][cols ? cols[k] : k] = (sum over groups of `group` slots, in order, each
+// the sum of its slots in order) / scale, k < k0.  A column index outside
+// [0, k0) is clamped into it.  Bound: HBM and the Infinity Cache (51 partials
+// of 1.3 MB for a 180,224-row minibatch); eight loads in flight per thread.
+__global__ __launch_bounds__(256) void l1_grad_reduce(const qqt_l1_grad_args a, int slots, int group,
                                                       int ws_cols, const int64_t* cols) {
   const int i = blockIdx.x * 256 + threadIdx.x;
   if (i >= HID * a.k0) return;
@@ -239,16 +310,24 @@ __global__ __launch_bounds__(256) void l1_grad_reduce(const qqt_l1_grad_args a, 
   const size_t pitch = (size_t)HID * ws_cols;
   const float* p = a.workspace + (size_t)h * ws_cols + k;
   const int64_t col = cols ? min(max(cols[k], (int64_t)0), (int64_t)a.k0 - 1) : (int64_t)k;
-  float sum = 0.0f;
-  int c = 0;
-  for (; c + 8 <= chunks; c += 8, p += 8 * pitch) {
+  float sum = 0.0f, part = 0.0f;
+  int at = 0, c = 0;                  // at: slots that the current group has taken
+  auto add = [&](float v) {
+    part = at == 0 ? v : part + v;
+    if (++at == group) {
+      sum += part;
+      at = 0;
+    }
+  };
+  for (; c + 8 <= slots; c += 8, p += 8 * pitch) {
     float v[8];
 #pragma unroll
     for (int j = 0; j < 8; ++j) v[j] = p[j * pitch];
 #pragma unroll
-    for (int j = 0; j < 8; ++j) sum += v[j];
+    for (int j = 0; j < 8; ++j) add(v[j]);
   }
-  for (; c < chunks; ++c, p += pitch) sum += *p;
+  for (; c < slots; ++c, p += pitch) add(*p);
+  if (at) sum += part;
   a.dw0[(size_t)h * a.k0 + col] = sum * inv;
 }
 
@@ -275,25 +354,50 @@ __global__ __launch_bounds__(256) void w0_pack_kernel(const float* w, const int6
   *reinterpret_cast<half8*>(out + 8 * (size_t)i) = v;
 }
 
-// Chunks of the batch: rows per chunk a multiple of KS, at least min_rows, and
-// chunks x column tiles at most TARGET_WGS (all workgroups resident at once,
+// Pieces of the batch: rows of each a multiple of KS, at least min_rows, and
+// pieces x column tiles at most TARGET_WGS (all workgroups resident at once,
 // one per CU) and MAX_CHUNKS: a 180,224-row minibatch of 2366 columns makes 51
-// chunks x 5 tiles.
-__host__ inline void plan(int batch, int k0, int min_rows, int& chunks, int& chunk_rows) {
+// pieces x 5 tiles.
+__host__ inline int pieces(int batch, int k0, int min_rows, int& rows) {
   const int tiles = (k0 + NCOL - 1) / NCOL;
-  chunks = (batch + min_rows - 1) / min_rows;
-  if (chunks > TARGET_WGS / tiles) chunks = TARGET_WGS / tiles;
-  if (chunks > MAX_CHUNKS) chunks = MAX_CHUNKS;
-  if (chunks < 1) chunks = 1;
-  chunk_rows = (batch + chunks - 1) / chunks;
-  chunk_rows = (chunk_rows + KS - 1) / KS * KS;
-  chunks = (batch + chunk_rows - 1) / chunk_rows;
+  int n = (batch - 1) / min_rows + 1;
+  if (n > TARGET_WGS / tiles) n = TARGET_WGS / tiles;
+  if (n > MAX_CHUNKS) n = MAX_CHUNKS;
+  if (n < 1) n = 1;
+  rows = (batch - 1) / n + 1;
+  rows = (rows - 1) / KS * KS + KS;
+  return (batch - 1) / rows + 1;
 }
 
-__host__ inline int64_t plan_floats(int batch, int k0, int min_rows) {
-  int chunks, rows;
-  plan(batch, k0, min_rows, chunks, rows);
-  return (int64_t)chunks * HID * ((k0 + NCOL - 1) / NCOL) * NCOL;
+// The order of the sums follows the batch and k0 alone: chunks of at least
+// CHUNK_ROWS rows, each a product of its own; groups of consecutive chunks,
+// each summed in chunk order; the groups summed in order.  There are at most as
+// many groups as the documented workspace (SLOT_ROWS) has slots.  A workspace
+// that holds every chunk's partial gives each chunk its own workgroups and
+// leaves both sums to the reduction; in a smaller one a slot's workgroups, of
+// the narrow tile, walk its group's chunks and add as they go.  Below 512 rows a
+// chunk's partial tiles (1.3 MB out and back) cost what the shorter walk saves.
+// With the reduction, 2366 columns, in the documented workspace (one chunk per
+// slot, wide tile -> groups) and in the preferred one: 8,192 rows 134 -> 60 and
+// 45 us, 45,056 rows 142 -> 115 and 90 us.
+struct Plan {
+  int chunks, rows, group;
+};
+__host__ inline Plan plan(int batch, int k0) {
+  Plan p;
+  int slot_rows;
+  const int slots = pieces(batch, k0, SLOT_ROWS, slot_rows);
+  p.chunks = pieces(batch, k0, CHUNK_ROWS, p.rows);
+  if (p.chunks <= slots + slots / 8) {     // a few chunks more are not worth walking
+    p.chunks = slots;
+    p.rows = slot_rows;
+  }
+  p.group = (p.chunks + slots - 1) / slots;
+  return p;
+}
+
+__host__ inline int64_t slot_floats(int k0) {
+  return (int64_t)HID * ((k0 + NCOL - 1) / NCOL) * NCOL;
 }
 
 }  // namespace l1g
@@ -342,13 +446,14 @@ extern "C" {
 int64_t qqt_l1_grad_workspace_floats(int32_t batch, int32_t k0) {
   using namespace qqt::l1g;
   if (batch <= 0 || k0 <= 0) return -1;
-  return plan_floats(batch, k0, MIN_CHUNK_ROWS);
+  int rows;
+  return pieces(batch, k0, SLOT_ROWS, rows) * slot_floats(k0);
 }
 
 int64_t qqt_l1_grad_preferred_floats(int32_t batch, int32_t k0) {
   using namespace qqt::l1g;
   if (batch <= 0 || k0 <= 0) return -1;
-  return plan_floats(batch, k0, FINE_CHUNK_ROWS);
+  return plan(batch, k0).chunks * slot_floats(k0);
 }
 
 namespace {
@@ -391,24 +496,24 @@ int l1_grad_workspace_check(const qqt_l1_grad_args& a, const char* who) {
 int l1_grad_launch(const qqt_l1_grad_args& a, hipStream_t st, const int64_t* cols = nullptr) {
   using namespace qqt;
   using namespace qqt::l1g;
-  // Finer chunks where the workspace holds them: chunks of 2048 rows leave an
-  // 8192-row batch on 20 workgroups (136 us with its reduction; 35 us in 16
-  // chunks of 512).  Below 512 rows the partial tiles (1.3 MB per chunk out
-  // and back) cost what the shorter walk saves.
-  int chunks, rows;
-  plan(a.batch, a.k0,
-       a.workspace_floats >= plan_floats(a.batch, a.k0, FINE_CHUNK_ROWS) ? FINE_CHUNK_ROWS
-                                                                         : MIN_CHUNK_ROWS,
-       chunks, rows);
-  const int tiles = (a.k0 + NCOL - 1) / NCOL;
-  const int ws_cols = tiles * NCOL;
-  QQT_LAUNCH(QQT_KERNEL_L1GRAD, l1_grad_kernel, dim3(tiles, chunks), dim3(NT), st, a, rows,
-             ws_cols);
+  const Plan p = plan(a.batch, a.k0);
+  const bool whole = a.workspace_floats >= p.chunks * slot_floats(a.k0);
+  const int per_slot = whole ? 1 : p.group;
+  const int slots = (p.chunks - 1) / per_slot + 1;
+  const bool narrow = per_slot > 1;
+  const int ncol = narrow ? NARROW : NCOL;
+  const int tiles = (a.k0 + ncol - 1) / ncol, ws_cols = tiles * ncol;
+  if (narrow)
+    QQT_LAUNCH(QQT_KERNEL_L1GRAD, l1_grad_kernel<NARROW>, dim3(tiles, slots), dim3(NT), st, a,
+               p.chunks, p.rows, ws_cols, per_slot);
+  else
+    QQT_LAUNCH(QQT_KERNEL_L1GRAD, l1_grad_kernel<NCOL>, dim3(tiles, slots), dim3(NT), st, a,
+               p.chunks, p.rows, ws_cols, per_slot);
   hipError_t err = hipGetLastError();
   if (err == hipSuccess) {
     const int n = HID * a.k0;
     QQT_LAUNCH(QQT_KERNEL_L1GRAD, l1_grad_reduce, dim3((n + 255) / 256), dim3(256), st, a,
-               chunks, ws_cols, cols);
+               slots, whole ? p.group : 1, ws_cols, cols);
     err = hipGetLastError();
   }
   if (err != hipSuccess) {
@@ -478,7 +583,7 @@ int qqt_l1_grad_noalloc(const qqt_l1_grad_args* a, void* stream) {
   if (!ptr) return QQT_E_LAUNCH;
   qqt_l1_grad_args b = *a;          // the caller's workspace fields are ignored
   b.workspace = ptr;
-  b.workspace_floats = qqt_l1_grad_workspace_floats(b.batch, b.k0);
+  b.workspace_floats = qqt_l1_grad_preferred_floats(b.batch, b.k0);
   if (b.workspace_floats > (int64_t)l1g::MAX_CHUNKS * l1g::HID * QQT_L1_GRAD_NOALLOC_MAX_K0) {
     snprintf(g_err, sizeof(g_err), "qqt_l1_grad_noalloc: plan exceeds the static scratch");
     return QQT_E_ARG;

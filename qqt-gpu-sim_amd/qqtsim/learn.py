@@ -204,7 +204,7 @@ class HipMlpActorCritic(nn.Module):
             scale = torch.exp2(torch.clamp(14.0 - torch.ceil(torch.log2(amax)), -100.0, 100.0))
         dw0 = torch.empty((HID, self.k0), dtype=torch.float32, device=x16.device)
         a.batch, a.k0, a.obs_stride = b, self.k0, x16.stride(0)
-        a.workspace_floats = need            # the plan follows it, not the buffer's history
+        a.workspace_floats = self._ws.numel()
         a.obs, a.dz1, a.dz_scale = x16.data_ptr(), dz1.data_ptr(), scale.data_ptr()
         a.workspace, a.dw0 = self._ws.data_ptr(), dw0.data_ptr()
         _capi.check(self._lib.qqt_l1_grad_columns(a, self._perm[pid].data_ptr(),

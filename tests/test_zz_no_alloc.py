@@ -96,3 +96,36 @@ def test_no_alloc_rejects_wider_observation(dev):
     a = _args(x16, dz1, torch.ones(1, device=dev), out, k0=2562)
     with pytest.raises(ValueError, match="exceeds the static scratch"):
         _capi.check(lib.qqt_l1_grad_noalloc(a, _capi.stream_handle(dev)))
+
+
+@pytest.mark.parametrize("b,k0", [(1_021, K0), (3_001, K0), (8_192, K0), (26_113, K0),
+                                  (60_000, K0), (5_000, 686)])
+def test_the_result_does_not_depend_on_the_workspace(dev, b, k0):
+    """The documented workspace (whose workgroups walk several chunks and add
+    as they go), the preferred one, a larger one, one just short of the
+    preferred and the static scratch: the same bits."""
+    from qqtsim import _capi
+
+    lib = _capi.lib()
+    x16, dz1, scale = _inputs(b, b, dev)
+
+    def run(floats):
+        out = torch.full((128, k0), float("nan"), dtype=torch.float32, device=dev)
+        a = _args(x16, dz1, scale, out, k0)
+        if floats is None:
+            _capi.check(lib.qqt_l1_grad_noalloc(a, _capi.stream_handle(dev)))
+        else:
+            ws = torch.full((floats,), float("nan"), dtype=torch.float32, device=dev)
+            a.workspace, a.workspace_floats = ws.data_ptr(), floats
+            _capi.check(lib.qqt_l1_grad(a, _capi.stream_handle(dev)))
+        torch.cuda.synchronize()
+        return out
+
+    need = lib.qqt_l1_grad_workspace_floats(b, k0)
+    best = lib.qqt_l1_grad_preferred_floats(b, k0)
+    want = run(need)
+    exact = dz1.double().t() @ x16[:, :k0].double()
+    # the split holds 22 bits of max |dz1|: 128 x k0 sums of b products
+    assert float((want - exact).norm()) <= 2e-6 * float(exact.norm())
+    for floats in (best, max(need, best - 1), 3 * best, None):
+        assert torch.equal(run(floats), want), floats
