@@ -12,7 +12,8 @@
 // tile, which keeps the result within ~1e-6 relative of a float32 sum.
 //
 // Grid: (column tile of 512 observation columns) x (chunk of the batch); tiles of
-// 128 columns where the workspace has slots for groups of chunks only (Plan).  A
+// 128 columns where the workspace has slots for groups of chunks only (Plan) or
+// the grid is small (l1_grad_launch).  A
 // workgroup (8 wavefronts, one per CU) owns a 128 x 512 float32 output tile
 // for its chunk, 64 x 128 per wavefront in registers, and walks the chunk 32
 // rows at a time.  Each step's 32 KB of observation and 16 KB of dz1 are
@@ -53,7 +54,7 @@ typedef float floatx4 __attribute__((ext_vector_type(4)));
 
 constexpr int HID = 128;          // first-layer outputs
 constexpr int NCOL = 512;         // observation columns per workgroup ...
-constexpr int NARROW = 128;       // ... and where its slot takes several chunks
+constexpr int NARROW = 128;       // ... and where its slot takes several chunks or the grid is small
 constexpr int KS = 32;            // batch rows per step (one MFMA K)
 // LDS row strides (halves; NC + 16 for the observation), 8 banks apart per row:
 // 16-byte stores and the transposing reads (4 rows of 32 bytes per 16 lanes)
@@ -379,7 +380,7 @@ __host__ inline int pieces(int batch, int k0, int min_rows, int& rows) {
 // chunk's partial tiles (1.3 MB out and back) cost what the shorter walk saves.
 // With the reduction, 2366 columns, in the documented workspace (one chunk per
 // slot, wide tile -> groups) and in the preferred one: 8,192 rows 134 -> 60 and
-// 45 us, 45,056 rows 142 -> 115 and 90 us.
+// 32 us, 45,056 rows 142 -> 115 and 90 us.
 struct Plan {
   int chunks, rows, group;
 };
@@ -500,7 +501,13 @@ int l1_grad_launch(const qqt_l1_grad_args& a, hipStream_t st, const int64_t* col
   const bool whole = a.workspace_floats >= p.chunks * slot_floats(a.k0);
   const int per_slot = whole ? 1 : p.group;
   const int slots = (p.chunks - 1) / per_slot + 1;
-  const bool narrow = per_slot > 1;
+  // The narrow tile also where the wide ones would leave three eighths of the
+  // CUs idle: a step of 32 rows takes a workgroup of the wide tile four times
+  // the products.  Wide and narrow, with the reduction, in the preferred
+  // workspace: 2366 columns, 1 row 11.4 and 7.4 us, 512 rows (5 wide tiles) 39
+  // and 18, 8,192 (80) 45 and 32, 20,000 (200) 52 and 55, 45,056 (255) 90 and
+  // 101; 686 columns, 45,056 rows (128) 55 and 49, 180,224 (128) 187 and 151.
+  const bool narrow = per_slot > 1 || (a.k0 + NCOL - 1) / NCOL * slots * 8 <= TARGET_WGS * 5;
   const int ncol = narrow ? NARROW : NCOL;
   const int tiles = (a.k0 + ncol - 1) / ncol, ws_cols = tiles * ncol;
   if (narrow)

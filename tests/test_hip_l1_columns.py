@@ -69,3 +69,29 @@ def test_bad_arguments_are_refused():
     for cols in (None, 4100):
         assert lib.qqt_l1_grad_columns(ctypes.byref(a), cols, None) == -1
         assert b"cols must be" in lib.qqt_last_error()
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("b,k0", [(1, 126), (31, 128), (33, 130), (513, 2432), (8192, 2560),
+                                  (9000, 258), (70_001, 1024), (70_001, 1026)])
+def test_narrow_and_wide_column_tiles(b, k0):
+    """Edges of the 128- and 512-column tiles and both sides of the rule that
+    picks them (1024 columns in 64 chunks: 128 wide tiles; 1026: 192), against
+    float64.  float16 pairs of a gradient scaled to 2^14 hold 22 bits."""
+    from qqtsim import _capi
+
+    lib, dev = _capi.lib(), torch.device("cuda:0")
+    g = torch.Generator(device=dev).manual_seed(b + k0)
+    x = (torch.rand((b, k0 + 2), generator=g, device=dev) < 0.2).half()[:, :k0]
+    dz = torch.randn((b, 128), generator=g, device=dev)
+    scale = torch.exp2(13.0 - torch.ceil(torch.log2(dz.abs().max()))).reshape(1)
+    cols = torch.arange(k0, device=dev)
+    need = int(lib.qqt_l1_grad_preferred_floats(b, k0))
+    ws, out = torch.empty(need, device=dev), torch.full((128, k0), float("nan"), device=dev)
+    a = _capi.L1GradArgsC()
+    a.batch, a.k0, a.obs_stride, a.workspace_floats = b, k0, k0 + 2, need
+    a.obs, a.dz1, a.dz_scale = x.data_ptr(), dz.data_ptr(), scale.data_ptr()
+    a.workspace, a.dw0 = ws.data_ptr(), out.data_ptr()
+    _capi.check(lib.qqt_l1_grad_columns(a, cols.data_ptr(), _capi.stream_handle(dev)))
+    want = dz.double().t() @ x.double()
+    assert float((out - want).norm()) <= 2e-6 * float(want.norm())
