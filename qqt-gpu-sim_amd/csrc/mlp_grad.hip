@@ -38,6 +38,7 @@
 #include <stdio.h>
 
 #include <mutex>
+#include <type_traits>
 
 #include "qqt_common.h"
 #include "qqt_hip.h"
@@ -119,8 +120,9 @@ __device__ __forceinline__ void l1_grad_chunk(const qqt_l1_grad_args& a, Lds<NC>
 
   // loader roles: wavefront w brings rows 4w .. 4w + 3 of the observation,
   // lane l columns 8 (l % LPR) .. + 7 of row l / LPR of each load; thread t row
-  // t / 16 of dz1, hidden 8 (t % 16) .. + 7.  Rows past the chunk: its last row
-  // again, against zero gradients.
+  // t / 16 of dz1, hidden 8 (t % 16) .. + 7.  Rows past the chunk load its last
+  // row again and are stored as zeros on both sides (an infinity or NaN of that
+  // row against a zero gradient would be NaN).
   const int dr = t >> 4, dc = 8 * (t & 15);
   struct Regs {
     u32x4 x[NL];
@@ -162,11 +164,17 @@ __device__ __forceinline__ void l1_grad_chunk(const qqt_l1_grad_args& a, Lds<NC>
     }
     __builtin_memcpy(g.d, a.dz1 + (size_t)min(r0 + dr, r_end - 1) * HID + dc, 32);
   };
-  auto store = [&](const Regs& g, int buf, int step) {
-    const bool live = r_begin + KS * step + dr < r_end;
+  // (end: the step may reach past the chunk)
+  auto store = [&](const Regs& g, int buf, int step, auto end) {
+    const int r0 = r_begin + KS * step;
+    const bool live = !decltype(end)::value || r0 + dr < r_end;
 #pragma unroll
-    for (int i = 0; i < NL; ++i)
-      *reinterpret_cast<u32x4*>(&s.x[buf][4 * w + RPL * i + lane / LPR][8 * (lane % LPR)]) = g.x[i];
+    for (int i = 0; i < NL; ++i) {
+      const int r = 4 * w + RPL * i + lane / LPR;
+      u32x4 x = g.x[i];
+      if (decltype(end)::value && r0 + r >= r_end) x = u32x4{0, 0, 0, 0};
+      *reinterpret_cast<u32x4*>(&s.x[buf][r][8 * (lane % LPR)]) = x;
+    }
     half8 hi, lo;
 #pragma unroll
     for (int k = 0; k < 8; ++k) {
@@ -219,29 +227,37 @@ __device__ __forceinline__ void l1_grad_chunk(const qqt_l1_grad_args& a, Lds<NC>
   // Register ring of two steps in flight beside the LDS double buffer: step i
   // computes from buffer i & 1, stores step i + 1 to the other and loads step
   // i + 3 into the slot that freed (steps past the last reload the last).
+  // Only the last step can reach past the chunk, and it is not stored in the loop.
   Regs g[2];
   const int last = steps - 1;
+  const std::integral_constant<bool, true> may_end;
+  const std::integral_constant<bool, false> whole;
   index(0);
   load(0, g[0]);
   load(min(1, last), g[1]);
-  store(g[0], 0, 0);
+  store(g[0], 0, 0, may_end);
   load(min(2, last), g[0]);
   __syncthreads();
   int i = 0;
-  for (; i + 2 <= last; i += 2) {
+  for (; i + 2 < last; i += 2) {
 #pragma unroll
     for (int k = 0; k < 2; ++k) {
       compute(k);
-      store(g[1 - k], 1 - k, i + k + 1);
+      store(g[1 - k], 1 - k, i + k + 1, whole);
       load(min(i + k + 3, last), g[1 - k]);
       __syncthreads();
     }
   }
   compute(0);
   if (i < last) {
-    store(g[1], 1, last);
+    store(g[1], 1, i + 1, may_end);
     __syncthreads();
     compute(1);
+    if (i + 1 < last) {
+      store(g[0], 0, last, may_end);
+      __syncthreads();
+      compute(0);
+    }
   }
 }
 
@@ -253,7 +269,7 @@ __device__ __forceinline__ void l1_grad_chunk(const qqt_l1_grad_args& a, Lds<NC>
 // against 294; tiles of 256 columns, two workgroups per CU, 317 us.  Adding a
 // slot's chunks in the workspace instead, which the wide tile would need, took
 // 232 us for 8,192 rows in four slots.)  The narrow tile is held to 128 registers
-// (13 go to scratch): two workgroups per CU take 45,056 rows in 17 slots in
+// (7 go to scratch): two workgroups per CU take 45,056 rows in 17 slots in
 // 115 us, one (156 registers) in 134.
 template <int NC, bool EDGE>
 __device__ __forceinline__ void l1_grad_slot(const qqt_l1_grad_args& a, Lds<NC>& s, int chunks,

@@ -95,3 +95,31 @@ def test_narrow_and_wide_column_tiles(b, k0):
     _capi.check(lib.qqt_l1_grad_columns(a, cols.data_ptr(), _capi.stream_handle(dev)))
     want = dz.double().t() @ x.double()
     assert float((out - want).norm()) <= 2e-6 * float(want.norm())
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("b,k0", [(1, 130), (33, 2366), (30_001, 2366)])
+def test_a_non_finite_last_row_stays_its_own(b, k0):
+    """An infinity and a NaN in the batch's last row reach dW0 as that row's
+    products alone: infinite with the gradient's sign, NaN where the entry is
+    NaN, the other columns finite (both column tiles; the last step of the
+    batch is partial).  That row's gradients have a high and a low part of one
+    sign, whose two products of an infinity do not cancel."""
+    from qqtsim import _capi
+
+    lib, dev = _capi.lib(), torch.device("cuda:0")
+    g = torch.Generator(device=dev).manual_seed(b)
+    x = (torch.rand((b, k0), generator=g, device=dev) < 0.2).half()
+    x[-1, 1], x[-1, 3], x[-1, k0 - 1] = float("inf"), float("nan"), float("-inf")
+    dz = torch.randn((b, 128), generator=g, device=dev)
+    dz[-1] = (1.0 + 2.0 ** -12) * dz[-1].sign()
+    need = int(lib.qqt_l1_grad_preferred_floats(b, k0))
+    ws, out = torch.empty(need, device=dev), torch.empty((128, k0), device=dev)
+    a = _capi.L1GradArgsC()
+    a.batch, a.k0, a.obs_stride, a.workspace_floats = b, k0, k0, need
+    a.obs, a.dz1, a.workspace, a.dw0 = (t.data_ptr() for t in (x, dz, ws, out))
+    _capi.check(lib.qqt_l1_grad(a, _capi.stream_handle(dev)))
+    assert torch.equal(out[:, 1], float("inf") * dz[-1].sign())
+    assert torch.equal(out[:, k0 - 1], -float("inf") * dz[-1].sign())
+    assert bool(out[:, 3].isnan().all())
+    assert torch.isfinite(out).all(0).sum() == k0 - 3
