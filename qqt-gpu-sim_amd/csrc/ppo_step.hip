@@ -10,10 +10,10 @@
 // passes it at its bounds); then the backward down to dz1.  Out come dz1, the
 // gradients of all parameters above W0 (b0 included) and the statistics.
 //
-// Bound: the matrix cores and the row phases' VALU work between barriers;
-// bytes are small (z1 in, dz1 out: 1 KB per row).  122,880 multiply-adds per
-// row (forward, input gradients, weight gradients), as three float16 products
-// each (below): 0.37 M per row.
+// Bound: the matrix cores, the row phases' VALU work and the operand reads
+// between barriers; bytes are small (z1 in, dz1 out: 1 KB per row).  122,880
+// multiply-adds per row (forward, input gradients, weight gradients), as six
+// bfloat16 products each (below): 0.74 M per row.
 //
 // Shape: persistent workgroups (one per CU, 8 wavefronts) walk 32-row tiles.
 // The activations of a tile live in LDS, the weight-gradient accumulators
@@ -22,23 +22,27 @@
 // goes to HBM; a row-output kernel followed by batched products moved 4.2 KB
 // per row out and 3.5 KB back in.  Partial sums go to the workspace once per
 // workgroup and ppo_finish_kernel adds them in workgroup order
-// (deterministic).  Measured on a 180,224-row minibatch: 304 us with 24 us of
+// (deterministic).  Measured on a 180,224-row minibatch: 401 us with 18 us of
 // packing and reduction beside it, where the row-output kernel (float32 MFMA),
-// its batched products, reductions and copies took 860 us; 29 k cycles per
-// 32-row tile (output and loss phase 4.5 k, LayerNorm backwards 4.6 k, the two
-// backward product phases 5.1 k, dhy 2.3 k, barriers 6.6 k).
+// its batched products, reductions and copies took 860 us.
 //
-// Products: v_mfma_f32_16x16x32_f16 on float16 hi/lo pairs, x = hi + lo, sum
-// hi hi + hi lo + lo hi (+ lo lo in the data products) in float32.  Every operand is scaled by a
-// power of two that puts its largest magnitude near 2^13 (weights: their
-// largest entry, found when they are packed; LayerNorm outputs: sqrt(127)
-// max|gamma| + max|beta|; the gradients: running scales per workgroup, one per
-// head for dhy and one for dz2, that only fall, with the accumulators
-// rescaled, exactly, when they do), so hi + lo holds 22-23 bits of every
-// operand that matters and nothing overflows.  Errors against float64 from the
-// same z1 (relative, start = the float32 MFMA kernel): one row 2.7e-7 (start
-// 3.4e-7), 16,398 rows dW1 1.1e-7 (1.3e-7), dWh 0.7-1.1e-7 (1.1-1.3e-7), bias
-// and LayerNorm sums 1.0-1.3e-7 (0.7e-7), 45,056 rows 0.9-1.4e-7 (0.9-3.5e-7).
+// Products: v_mfma_f32_16x16x32_bf16 on three bfloat16 pieces of each operand,
+// x = x0 + x1 + x2, which hold float32's 24 bits at any magnitude: a row or a
+// weight keeps its precision whatever stands beside or before it, with no
+// scales.  The sum takes x0 y0, x0 y1, x1 y0, x1 y1, x0 y2 and x2 y0; the three
+// left out are below 2^-25 of x y.  In the data products the leading product
+// has an accumulator of its own (one rounding of the whole sum per 32
+// features).  (float16 pairs under running power-of-two scales, four products,
+// took 305 us and held 22 bits of each workgroup's largest row: rows of 1e-9
+// of it lost all of dz1, and the bias and LayerNorm sums of 8,192 rows were 1.3
+// to 1.6 times as far from float64 as the float32 kernel's.)  Errors against
+// float64 from the same z1, geometric means over three kinds of data, the
+// row-output float32 kernel -> this one: 1 to 1,021 rows dW1 1.8e-7 -> 1.1e-7,
+// dWh 1.5-2.4e-7 -> 0.9-1.6e-7, bias and LayerNorm sums 0.6-1.9e-7 -> 0.4-1.3e-7;
+// 1 to 180,224 rows dW1 1.4e-7 -> 0.7e-7, dWh 1.1-2.2e-7 -> 0.6-1.3e-7, sums
+// 0.5-1.3e-7 -> 0.3-1.1e-7; the worst dz1 row of 40,001 that span nine orders of
+// magnitude 8.7e-7 -> 6.7e-7.
+//
 // Data products contract over features (8 consecutive features of a row per
 // lane); weight gradients contract over the tile's 32 rows, the same LDS rows
 // read through the transposing ds_read_b64_tr_b16.
@@ -71,14 +75,14 @@ constexpr int HS = H + 16, YS = HY + 16;
 constexpr int XS = H + 4, HYS = HY + 4;     // float rows
 constexpr float LN_EPS = 1e-5f;
 
-// weight fragments of the workspace (halves): [tile][K step][plane][lane][8]
-constexpr int FRAG = 512;                    // halves of one (tile, step, plane)
+// weight fragments of the workspace (values): [tile][K step][piece][lane][8]
+constexpr int FRAG = 512;                    // values of one (tile, step, piece)
 constexpr int F_Z2 = 0;                      // W1,   8 tiles x 4 steps: z2 = W1 h1
-constexpr int F_HY = F_Z2 + 8 * 4 * 2 * FRAG;    // Wh,  12 x 4: hy = Wh h2
-constexpr int F_DH2 = F_HY + 12 * 4 * 2 * FRAG;  // Wh^T, 8 x 6: dh2 = Wh^T dhy
-constexpr int F_DH1 = F_DH2 + 8 * 6 * 2 * FRAG;  // W1^T, 8 x 4: dh1 = W1^T dz2
-constexpr int F_END = F_DH1 + 8 * 4 * 2 * FRAG;
-constexpr int N_FRAGS = F_END / (2 * FRAG) * 64;   // (tile, step, lane) items of the pack kernel
+constexpr int F_HY = F_Z2 + 8 * 4 * 3 * FRAG;    // Wh,  12 x 4: hy = Wh h2
+constexpr int F_DH2 = F_HY + 12 * 4 * 3 * FRAG;  // Wh^T, 8 x 6: dh2 = Wh^T dhy
+constexpr int F_DH1 = F_DH2 + 8 * 6 * 3 * FRAG;  // W1^T, 8 x 4: dh1 = W1^T dz2
+constexpr int F_END = F_DH1 + 8 * 4 * 3 * FRAG;
+constexpr int N_FRAGS = F_END / (3 * FRAG) * 64;   // (tile, step, lane) items of the pack kernel
 
 // one workgroup's partial sums (floats)
 constexpr int P_W1 = 0, P_WH = P_W1 + H * H, P_WF = P_WH + HY * H, P_G1 = P_WF + 8 * 64,
@@ -87,16 +91,19 @@ constexpr int P_W1 = 0, P_WH = P_W1 + H * H, P_WF = P_WH + HY * H, P_G1 = P_WF +
               P_MX = P_ST + 5, P_N = P_MX + 1;
 constexpr int P_PAD = (P_N + 63) / 64 * 64;
 
-// workspace: fragments | scales (W1, Wh) | partials
-constexpr size_t WS_SCALE = (size_t)F_END * 2;
-constexpr size_t WS_PART = WS_SCALE + 256;
+// workspace: fragments | partials
+constexpr size_t WS_PART = (size_t)F_END * 2;
 
+typedef __bf16 bf8 __attribute__((ext_vector_type(8)));
+typedef float float8v __attribute__((ext_vector_type(8)));
 typedef short s4 __attribute__((ext_vector_type(4)));
 typedef __attribute__((address_space(3))) s4 lds_s4;
 
 struct __align__(16) Lds {
-  uint16_t h1[2][R][HS], h2[2][R][HS];      // hi | lo planes of h1, h2
-  uint16_t dy[2][R][YS], dz[2][R][HS];      // ... of dhy, dz2
+  uint16_t h1[3][R][HS], h2[3][R][HS];      // pieces of h1, h2
+  union {                                   // ... of dhy, then of dz2
+    uint16_t dy[3][R][YS], dz[3][R][HS];
+  };
   float ex[R][XS];                          // z2, dh2, dh1 on their way to the row phases
   float hy[R][HYS];
   float dl[R][8];
@@ -104,7 +111,7 @@ struct __align__(16) Lds {
   float sum[3][R][16];                      // each thread's running output-gradient sum, statistic, max |dz1|
   float ln[4][H];                           // gamma1, beta1, gamma2, beta2
   float b1[H], bh[HY], wf[8][64], bf[8];
-  float dlmax[8][16], zred[8];              // per wavefront: max |dl| by lane of a row, max |dz2|
+  float mx[8];                              // per wavefront: max |dz1|
 };
 
 // 2^e for a clamped exponent
@@ -143,17 +150,27 @@ __device__ __forceinline__ float max64(float v) {
   return fmaxf(v, __shfl_xor(v, 32, 64));
 }
 
-__device__ __forceinline__ half8 ld8(const uint16_t* p) {
-  return as_h8(*reinterpret_cast<const uint4*>(p));
-}
+__device__ __forceinline__ bf8 ld8(const uint16_t* p) { return *reinterpret_cast<const bf8*>(p); }
 
-// Split eight scaled values into hi and lo, stored as 16 bytes per plane.
-__device__ __forceinline__ void split8(const float (&v)[8], uint16_t* hi, uint16_t* lo) {
-  half8 h, l;
+// The three bfloat16 pieces of eight values, v = p[0] + p[1] + p[2] (each the
+// nearest to what the ones before leave).
+__device__ __forceinline__ void split8(const float (&v)[8], bf8 (&p)[3]) {
+  float8v r;
 #pragma unroll
-  for (int i = 0; i < 8; ++i) split_into(v[i], h, l, i);
-  *reinterpret_cast<half8*>(hi) = h;
-  *reinterpret_cast<half8*>(lo) = l;
+  for (int i = 0; i < 8; ++i) r[i] = v[i];
+#pragma unroll
+  for (int k = 0; k < 3; ++k) {
+    p[k] = __builtin_convertvector(r, bf8);
+    if (k < 2) r -= __builtin_convertvector(p[k], float8v);
+  }
+}
+// ... to an LDS plane each
+template <int S>
+__device__ __forceinline__ void put8(const float (&v)[8], uint16_t (&plane)[3][R][S], int row, int at) {
+  bf8 p[3];
+  split8(v, p);
+#pragma unroll
+  for (int k = 0; k < 3; ++k) *reinterpret_cast<bf8*>(&plane[k][row][at]) = p[k];
 }
 
 // Transposed operand of a contraction over the tile's rows: element i of lane
@@ -161,26 +178,45 @@ __device__ __forceinline__ void split8(const float (&v)[8], uint16_t* hi, uint16
 // stride S.  One transposing read: lanes 4a..4a+3 of a 16-lane group address
 // row 8q + a (32 bytes), and lane j receives column j of those four rows.
 template <int S>
-__device__ __forceinline__ half8 ld_rows(const uint16_t* plane, int tile, int lane) {
+__device__ __forceinline__ bf8 ld_rows(const uint16_t (&plane)[R][S], int tile, int lane) {
   const int q = lane >> 4, j = lane & 15;
-  const uint16_t* p = plane + (8 * q + (j >> 2)) * S + 16 * tile + 4 * (j & 3);
+  const uint16_t* p = &plane[8 * q + (j >> 2)][16 * tile + 4 * (j & 3)];
   const s4 a = __builtin_amdgcn_ds_read_tr16_b64_v4i16((lds_s4*)(p));
   const s4 b = __builtin_amdgcn_ds_read_tr16_b64_v4i16((lds_s4*)(p + 4 * S));
-  return __builtin_bit_cast(half8, __builtin_shufflevector(a, b, 0, 1, 2, 3, 4, 5, 6, 7));
+  return __builtin_bit_cast(bf8, __builtin_shufflevector(a, b, 0, 1, 2, 3, 4, 5, 6, 7));
 }
 
-// c += (ah + al)(bh + bl): all four products where the result feeds the rest
-// of the chain; a weight gradient, summed over the batch, leaves out al bl
-__device__ __forceinline__ floatx4 mfma4(half8 ah, half8 al, half8 bh, half8 bl, floatx4 c) {
-  c = mfma(al, bl, c);
-  c = mfma(al, bh, c);
-  c = mfma(ah, bl, c);
-  return mfma(ah, bh, c);
+// c += a b without the three products below 2^-25 of it
+__device__ __forceinline__ floatx4 mfma6(const bf8 (&a)[3], const bf8 (&b)[3], floatx4 c) {
+  c = __builtin_amdgcn_mfma_f32_16x16x32_bf16(a[2], b[0], c, 0, 0, 0);
+  c = __builtin_amdgcn_mfma_f32_16x16x32_bf16(a[0], b[2], c, 0, 0, 0);
+  c = __builtin_amdgcn_mfma_f32_16x16x32_bf16(a[1], b[1], c, 0, 0, 0);
+  c = __builtin_amdgcn_mfma_f32_16x16x32_bf16(a[1], b[0], c, 0, 0, 0);
+  c = __builtin_amdgcn_mfma_f32_16x16x32_bf16(a[0], b[1], c, 0, 0, 0);
+  return __builtin_amdgcn_mfma_f32_16x16x32_bf16(a[0], b[0], c, 0, 0, 0);
 }
-__device__ __forceinline__ floatx4 mfma3(half8 ah, half8 al, half8 bh, half8 bl, floatx4 c) {
-  c = mfma(al, bh, c);
-  c = mfma(ah, bl, c);
-  return mfma(ah, bh, c);
+
+// The same with the leading products summed apart from the others (c[0], c[1]):
+// one rounding of the whole sum per step of 32 instead of six.
+__device__ __forceinline__ void mfma6(const bf8 (&a)[3], const bf8 (&b)[3], floatx4 (&c)[2]) {
+  c[1] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(a[2], b[0], c[1], 0, 0, 0);
+  c[1] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(a[0], b[2], c[1], 0, 0, 0);
+  c[0] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(a[0], b[0], c[0], 0, 0, 0);
+  c[1] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(a[1], b[1], c[1], 0, 0, 0);
+  c[1] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(a[1], b[0], c[1], 0, 0, 0);
+  c[1] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(a[0], b[1], c[1], 0, 0, 0);
+}
+
+// The pieces of eight consecutive features of a row.
+struct Pieces {
+  bf8 p[3];
+};
+template <int S>
+__device__ __forceinline__ Pieces ld_pieces(const uint16_t (&plane)[3][R][S], int row, int at) {
+  Pieces f;
+#pragma unroll
+  for (int n = 0; n < 3; ++n) f.p[n] = ld8(&plane[n][row][at]);
+  return f;
 }
 
 // Sum of each of the eight values over the wavefront's four 16-lane rows;
@@ -208,9 +244,9 @@ __device__ __forceinline__ void load8(const float* p, float (&v)[8]) {
 }
 
 // LayerNorm of a row over its 16 threads (8 values each): xh and 1/std, and
-// the scaled ReLU output's hi/lo planes.
+// the ReLU output.
 __device__ __forceinline__ void ln_forward(float (&z)[8], const float* gam, const float* bet,
-                                           float scale, float& rstd, uint16_t* hi, uint16_t* lo) {
+                                           float& rstd, float (&h)[8]) {
   float s = 0.0f;
 #pragma unroll
   for (int i = 0; i < 8; ++i) s += z[i];
@@ -222,15 +258,14 @@ __device__ __forceinline__ void ln_forward(float (&z)[8], const float* gam, cons
     d2 = __builtin_fmaf(z[i], z[i], d2);
   }
   rstd = 1.0f / sqrtf(sum16(d2) * (1.0f / H) + LN_EPS);
-  float g[8], b[8], h[8];
+  float g[8], b[8];
   load8(gam, g);
   load8(bet, b);
 #pragma unroll
   for (int i = 0; i < 8; ++i) {
     z[i] *= rstd;
-    h[i] = fmaxf(__builtin_fmaf(z[i], g[i], b[i]), 0.0f) * scale;
+    h[i] = fmaxf(__builtin_fmaf(z[i], g[i], b[i]), 0.0f);
   }
-  split8(h, hi, lo);
 }
 
 // Backward of LayerNorm + ReLU for a row's 16 threads: d = gradient of the
@@ -260,59 +295,29 @@ __device__ __forceinline__ float tree8(const float (&u)[8]) {
   return ((u[0] + u[1]) + (u[2] + u[3])) + ((u[4] + u[5]) + (u[6] + u[7]));
 }
 
-// Weights -> scaled hi/lo MFMA A fragments (element i of lane (r16, q) in K
+// Weights -> the pieces of their MFMA A fragments (element i of lane (r16, q) in K
 // step s of tile m: M[16 m + r16][32 s + 8 q + i], M = W1, Wh, Wh^T, W1^T).
-// Every workgroup finds the two scales itself (160 KB from L2).
 __global__ __launch_bounds__(256) void ppo_pack_kernel(const qqt_ppo_step_args a) {
-  __shared__ float red[2][4];
-  const int t = threadIdx.x;
-  const float4* w1v = reinterpret_cast<const float4*>(a.w1);
-  auto amax4 = [](float m, float4 v) {
-    return fmaxf(m, fmaxf(fmaxf(fabsf(v.x), fabsf(v.y)), fmaxf(fabsf(v.z), fabsf(v.w))));
-  };
-  // (all 40 loads in flight at once)
-  float4 v1[H * H / 4 / 256], vh[3 * 64 * H / 4 / 256];
-#pragma unroll
-  for (int i = 0; i < H * H / 4 / 256; ++i) v1[i] = w1v[t + 256 * i];
-#pragma unroll
-  for (int i = 0; i < 3 * 64 * H / 4 / 256; ++i)
-    vh[i] = reinterpret_cast<const float4*>(a.wh[i >> 3])[t + 256 * (i & 7)];
-  float m1 = 0.0f, mh = 0.0f;
-#pragma unroll
-  for (int i = 0; i < H * H / 4 / 256; ++i) m1 = amax4(m1, v1[i]);
-#pragma unroll
-  for (int i = 0; i < 3 * 64 * H / 4 / 256; ++i) mh = amax4(mh, vh[i]);
-  m1 = max64(m1);
-  mh = max64(mh);
-  if ((t & 63) == 0) {
-    red[0][t >> 6] = m1;
-    red[1][t >> 6] = mh;
-  }
-  __syncthreads();
-  const float s1 = scale_for(fmaxf(fmaxf(red[0][0], red[0][1]), fmaxf(red[0][2], red[0][3])));
-  const float sh = scale_for(fmaxf(fmaxf(red[1][0], red[1][1]), fmaxf(red[1][2], red[1][3])));
   uint16_t* const F = static_cast<uint16_t*>(a.workspace);
-  if (blockIdx.x == 0 && t < 2)
-    reinterpret_cast<float*>(static_cast<char*>(a.workspace) + WS_SCALE)[t] = t ? sh : s1;
-  const int item = blockIdx.x * 256 + t;            // (fragment, lane)
+  const int item = blockIdx.x * 256 + threadIdx.x;  // (fragment, lane)
   if (item >= N_FRAGS) return;
   const int f = item >> 6, lane = item & 63, r16 = lane & 15, q = lane >> 4;
   // fragments in workspace order: W1 (32), Wh (48), Wh^T (48), W1^T (32)
   const int part = f < 32 ? 0 : f < 80 ? 1 : f < 128 ? 2 : 3;
   const int g = f - (part == 0 ? 0 : part == 1 ? 32 : part == 2 ? 80 : 128);
   const int ks = part == 2 ? 6 : 4, m = 16 * (g / ks) + r16, k = 32 * (g % ks) + 8 * q;
-  half8 hi, lo;
+  float v[8];
 #pragma unroll
   for (int i = 0; i < 8; ++i) {
-    float v;
-    if (part == 0) v = a.w1[m * H + k + i];
-    else if (part == 1) v = a.wh[m >> 6][(m & 63) * H + k + i];
-    else if (part == 2) v = a.wh[(k + i) >> 6][((k + i) & 63) * H + m];
-    else v = a.w1[(k + i) * H + m];
-    split_into(v * (part == 0 || part == 3 ? s1 : sh), hi, lo, i);
+    if (part == 0) v[i] = a.w1[m * H + k + i];
+    else if (part == 1) v[i] = a.wh[m >> 6][(m & 63) * H + k + i];
+    else if (part == 2) v[i] = a.wh[(k + i) >> 6][((k + i) & 63) * H + m];
+    else v[i] = a.w1[(k + i) * H + m];
   }
-  *reinterpret_cast<half8*>(F + (size_t)f * 2 * FRAG + lane * 8) = hi;
-  *reinterpret_cast<half8*>(F + (size_t)f * 2 * FRAG + FRAG + lane * 8) = lo;
+  bf8 p[3];
+  split8(v, p);
+#pragma unroll
+  for (int n = 0; n < 3; ++n) *reinterpret_cast<bf8*>(F + (size_t)(3 * f + n) * FRAG + lane * 8) = p[n];
 }
 
 __global__ __launch_bounds__(T) void ppo_step_kernel(const qqt_ppo_step_args a, int tiles) {
@@ -332,15 +337,17 @@ __global__ __launch_bounds__(T) void ppo_step_kernel(const qqt_ppo_step_args a, 
     lane16 = lane * 16;
   };
   place();
-  const float* const wscale = reinterpret_cast<const float*>(static_cast<const char*>(a.workspace) + WS_SCALE);
   // weight fragments: one lane offset for all of them, the rest is scalar
   const Rsrc F = rsrc(a.workspace, F_END * 2);
-  auto frag = [&](int base, int ks, int tile, int step, int plane) {
-    const int at = 2 * (base + ((tile * ks + step) * 2 + plane) * FRAG);
-    return __builtin_bit_cast(half8, __builtin_amdgcn_raw_buffer_load_b128(F, lane16, at, 0));
+  auto frag = [&](bf8 (&f)[3], int base, int ks, int tile, int step) {
+#pragma unroll
+    for (int n = 0; n < 3; ++n) {
+      const int at = 2 * (base + ((tile * ks + step) * 3 + n) * FRAG);
+      f[n] = __builtin_bit_cast(bf8, __builtin_amdgcn_raw_buffer_load_b128(F, lane16, at, 0));
+    }
   };
 
-  // ---- parameters -> LDS; scales
+  // ---- parameters -> LDS
   if (t < H) {
     s.ln[0][t] = a.ln1_w[t];
     s.ln[1][t] = a.ln1_b[t];
@@ -355,29 +362,9 @@ __global__ __launch_bounds__(T) void ppo_step_kernel(const qqt_ppo_step_args a, 
   }
   if (t < 8) s.bf[t] = t < 5 ? a.bf[0][t] : t < 7 ? a.bf[1][t - 5] : a.bf[2][0];
   __syncthreads();
-  // |LayerNorm output| <= sqrt(H - 1) max|gamma| + max|beta|
-  auto bound = [&](const float* gam, const float* bet) {
-    const float g = max64(fmaxf(fabsf(gam[lane]), fabsf(gam[lane + 64])));
-    const float b = max64(fmaxf(fabsf(bet[lane]), fabsf(bet[lane + 64])));
-    return 11.27f * g + b;
-  };
-  const float sh1 = uniform(scale_for(bound(s.ln[0], s.ln[1])));
-  const float sh2 = uniform(scale_for(bound(s.ln[2], s.ln[3])));
-  const float sw1 = wscale[0], swh = wscale[1];
-  const float inv_z2 = uniform(1.0f / (sw1 * sh1)), inv_hy = uniform(1.0f / (swh * sh2));
   const float gmin = uniform(-1.0f / (float)a.batch);                          // d loss / d min_i
   const float gmax = uniform(a.value_coef * 0.5f / (float)a.batch);            // ... / d max_i
   const float gh = uniform(-a.entropy_coef / (float)a.batch);                  // ... / d entropy_i
-  // |dhy| of a head <= max|dl| max_f sum_o |wf[o][f]| over its outputs
-  float wcol[3];
-  {
-    float m = 0.0f;
-#pragma unroll
-    for (int k = 0; k < 5; ++k) m += fabsf(s.wf[k][lane]);
-    wcol[0] = uniform(max64(m));
-    wcol[1] = uniform(max64(fabsf(s.wf[5][lane]) + fabsf(s.wf[6][lane])));
-    wcol[2] = uniform(max64(fabsf(s.wf[7][lane])));
-  }
 
   // ---- accumulators of the whole launch
   floatx4 dwh[3][4], dw1[2][4];                  // feature tiles (3a + i | 2a + i) x (4b + n)
@@ -389,9 +376,6 @@ __global__ __launch_bounds__(T) void ppo_step_kernel(const qqt_ppo_step_args a, 
 #pragma unroll
     for (int i = 0; i < 2; ++i) dw1[i][n] = floatx4{0.0f, 0.0f, 0.0f, 0.0f};
   }
-  // running scales of dhy (each head its own: policy and value gradients
-  // differ by orders of magnitude) and dz2
-  float sy[3] = {0x1p100f, 0x1p100f, 0x1p100f}, sz = 0x1p100f;
   float dwf[8], dbh[3];
 #pragma unroll
   for (int o = 0; o < 8; ++o) dwf[o] = 0.0f;
@@ -432,12 +416,10 @@ __global__ __launch_bounds__(T) void ppo_step_kernel(const qqt_ppo_step_args a, 
     if (byte_in) lin = *reinterpret_cast<const uint8_t*>(p);
     else lin = *reinterpret_cast<const uint32_t*>(p);
   };
-  half8 wz[4][2];
+  bf8 wz[4][3];
   auto load_wz = [&]() {
 #pragma unroll
-    for (int k = 0; k < 4; ++k)
-#pragma unroll
-      for (int p = 0; p < 2; ++p) wz[k][p] = frag(F_Z2, 4, w, k, p);
+    for (int k = 0; k < 4; ++k) frag(wz[k], F_Z2, 4, w, k);
   };
   fetch(blockIdx.x);
   fetch_index(blockIdx.x);
@@ -450,36 +432,31 @@ __global__ __launch_bounds__(T) void ppo_step_kernel(const qqt_ppo_step_args a, 
     const int g = tile * R + row;
     const bool live = g < a.batch;
     // ---- LayerNorm 1 (rows past the batch: z1 = 0; their gradients are 0)
-    float x1[8], rs1;
+    float x1[8], rs1, hv[8];
 #pragma unroll
     for (int i = 0; i < 8; ++i) x1[i] = zn[i];
-    ln_forward(x1, s.ln[0] + 8 * j, s.ln[1] + 8 * j, sh1, rs1, &s.h1[0][row][8 * j], &s.h1[1][row][8 * j]);
+    ln_forward(x1, s.ln[0] + 8 * j, s.ln[1] + 8 * j, rs1, hv);
+    put8(hv, s.h1, row, 8 * j);
     fetch_index(tile + gridDim.x);
     __syncthreads();
 
     // ---- z2 = W1 h1 + b1: wavefront w, features 16w .. 16w + 15 of both row tiles
     {
-      floatx4 c[2] = {{0.0f, 0.0f, 0.0f, 0.0f}, {0.0f, 0.0f, 0.0f, 0.0f}};
+      floatx4 c[2][2] = {};                     // [row tile][leading | others]
 #pragma unroll
       for (int k = 0; k < 4; ++k)
 #pragma unroll
-        for (int rt = 0; rt < 2; ++rt) {
-          const int at = 32 * k + 8 * q;
-          c[rt] = mfma4(wz[k][0], wz[k][1], ld8(&s.h1[0][16 * rt + r16][at]),
-                        ld8(&s.h1[1][16 * rt + r16][at]), c[rt]);
-        }
+        for (int rt = 0; rt < 2; ++rt) mfma6(wz[k], ld_pieces(s.h1, 16 * rt + r16, 32 * k + 8 * q).p, c[rt]);
       const floatx4 b = *reinterpret_cast<const floatx4*>(&s.b1[16 * w + 4 * q]);
 #pragma unroll
       for (int rt = 0; rt < 2; ++rt)
-        *reinterpret_cast<floatx4*>(&s.ex[16 * rt + r16][16 * w + 4 * q]) = c[rt] * inv_z2 + b;
+        *reinterpret_cast<floatx4*>(&s.ex[16 * rt + r16][16 * w + 4 * q]) = (c[rt][1] + c[rt][0]) + b;
     }
     // head tiles w and 8 + w / 2: half before LayerNorm 2, half during it
-    half8 wy[4][2][2];
+    bf8 wy[4][2][3];
     auto load_wy = [&](int k) {
 #pragma unroll
-      for (int u = 0; u < 2; ++u)
-#pragma unroll
-        for (int p = 0; p < 2; ++p) wy[k][u][p] = frag(F_HY, 4, u ? 8 + (w >> 1) : w, k, p);
+      for (int u = 0; u < 2; ++u) frag(wy[k][u], F_HY, 4, u ? 8 + (w >> 1) : w, k);
     };
     load_wy(0);
     load_wy(1);
@@ -490,32 +467,27 @@ __global__ __launch_bounds__(T) void ppo_step_kernel(const qqt_ppo_step_args a, 
     load_wy(3);
     float x2[8], rs2;
     load8(&s.ex[row][8 * j], x2);
-    ln_forward(x2, s.ln[2] + 8 * j, s.ln[3] + 8 * j, sh2, rs2, &s.h2[0][row][8 * j], &s.h2[1][row][8 * j]);
+    ln_forward(x2, s.ln[2] + 8 * j, s.ln[3] + 8 * j, rs2, hv);
+    put8(hv, s.h2, row, 8 * j);
     __syncthreads();
 
-    // ---- heads' hidden layers: tile w for both row tiles, tile 8 + w / 2 for row tile w & 1
+    // ---- heads' hidden layers: tile w for both row tiles (w & 1 first), tile
+    // 8 + w / 2 for row tile w & 1
     {
-      floatx4 c[3];
-#pragma unroll
-      for (int u = 0; u < 3; ++u) c[u] = floatx4{0.0f, 0.0f, 0.0f, 0.0f};
+      floatx4 c[3][2] = {};
 #pragma unroll
       for (int k = 0; k < 4; ++k) {
-        const int at = 32 * k + 8 * q;
-        half8 bh[2], bl[2];
-#pragma unroll
-        for (int rt = 0; rt < 2; ++rt) {
-          bh[rt] = ld8(&s.h2[0][16 * rt + r16][at]);
-          bl[rt] = ld8(&s.h2[1][16 * rt + r16][at]);
-        }
-#pragma unroll
-        for (int rt = 0; rt < 2; ++rt) c[rt] = mfma4(wy[k][0][0], wy[k][0][1], bh[rt], bl[rt], c[rt]);
-        c[2] = mfma4(wy[k][1][0], wy[k][1][1], tb ? bh[1] : bh[0], tb ? bl[1] : bl[0], c[2]);
+        const Pieces b0 = ld_pieces(s.h2, 16 * tb + r16, 32 * k + 8 * q);
+        const Pieces b1 = ld_pieces(s.h2, 16 * (tb ^ 1) + r16, 32 * k + 8 * q);
+        mfma6(wy[k][0], b0.p, c[0]);
+        mfma6(wy[k][0], b1.p, c[1]);
+        mfma6(wy[k][1], b0.p, c[2]);
       }
 #pragma unroll
       for (int u = 0; u < 3; ++u) {
-        const int ft = u < 2 ? w : 8 + ta, rt = u < 2 ? u : tb;
+        const int ft = u < 2 ? w : 8 + ta, rt = u == 1 ? tb ^ 1 : tb;
         const floatx4 b = *reinterpret_cast<const floatx4*>(&s.bh[16 * ft + 4 * q]);
-        floatx4 v = c[u] * inv_hy + b;
+        floatx4 v = (c[u][1] + c[u][0]) + b;
 #pragma unroll
         for (int i = 0; i < 4; ++i) v[i] = fmaxf(v[i], 0.0f);
         *reinterpret_cast<floatx4*>(&s.hy[16 * rt + r16][16 * ft + 4 * q]) = v;
@@ -528,13 +500,14 @@ __global__ __launch_bounds__(T) void ppo_step_kernel(const qqt_ppo_step_args a, 
     {
       const float* y = &s.hy[row][64 * grp + 32 * part];
       const float* wo = &s.wf[o][32 * part];
-      float acc = 0.0f;
+      floatx4 part4 = {0.0f, 0.0f, 0.0f, 0.0f};          // four short chains round less
 #pragma unroll
       for (int k = 0; k < 32; k += 4) {
         const floatx4 yv = *reinterpret_cast<const floatx4*>(y + k), wv = *reinterpret_cast<const floatx4*>(wo + k);
 #pragma unroll
-        for (int i = 0; i < 4; ++i) acc = __builtin_fmaf(yv[i], wv[i], acc);
+        for (int i = 0; i < 4; ++i) part4[i] = __builtin_fmaf(yv[i], wv[i], part4[i]);
       }
+      float acc = (part4[0] + part4[1]) + (part4[2] + part4[3]);
       acc += __int_as_float(__builtin_amdgcn_update_dpp(0, __float_as_int(acc), 0xB1, 0xf, 0xf, true));
       const float logit = acc + s.bf[o];
       const float old_logp = __uint_as_float(s.in[row][0]), adv = __uint_as_float(s.in[row][1]);
@@ -580,16 +553,9 @@ __global__ __launch_bounds__(T) void ppo_step_kernel(const qqt_ppo_step_args a, 
       if (live)
         s.sum[1][row][j] += j == 0 ? -fminf(s1, s2) : j == 1 ? 0.5f * fmaxf(e1, e2) : j == 2 ? hm + hb
             : j == 3 ? old_logp - logp : fabsf(ratio - 1.0f) > a.clip_eps ? 1.0f : 0.0f;
-      float md = fabsf(d);
-      md = fmaxf(md, __shfl_xor(md, 16, 64));
-      md = fmaxf(md, __shfl_xor(md, 32, 64));
-      if (lane < 16) s.dlmax[w][lane] = md;
     }
-    half8 wd[6][2];
-    auto load_wd = [&](int k) {
-#pragma unroll
-      for (int p = 0; p < 2; ++p) wd[k][p] = frag(F_DH2, 6, w, k, p);
-    };
+    bf8 wd[6][3];
+    auto load_wd = [&](int k) { frag(wd[k], F_DH2, 6, w, k); };
 #pragma unroll
     for (int k = 0; k < 3; ++k) load_wd(k);
     __syncthreads();
@@ -599,22 +565,6 @@ __global__ __launch_bounds__(T) void ppo_step_kernel(const qqt_ppo_step_args a, 
 #pragma unroll
     for (int k = 3; k < 6; ++k) load_wd(k);
     {
-      float m = s.dlmax[0][j];
-#pragma unroll
-      for (int i = 1; i < 8; ++i) m = fmaxf(m, s.dlmax[i][j]);
-#pragma unroll
-      for (int h = 0; h < 3; ++h) {
-        const float mh = uniform(max16(grp == h ? m : 0.0f) * wcol[h]);
-        if (mh * sy[h] > 0x1p15f) {              // uniform over the workgroup
-          const float ns = uniform(scale_for(mh)), f = uniform(ns / sy[h]);
-          sy[h] = ns;
-#pragma unroll
-          for (int i = 0; i < 3; ++i)
-            if ((3 * ta + i) >> 2 == h)
-#pragma unroll
-              for (int n = 0; n < 4; ++n) dwh[i][n] *= f;
-        }
-      }
       float wfr[8];                              // output layer's column `lane` of each row
 #pragma unroll
       for (int k = 0; k < 8; ++k) wfr[k] = s.wf[k][lane];
@@ -642,51 +592,42 @@ __global__ __launch_bounds__(T) void ppo_step_kernel(const qqt_ppo_step_args a, 
         dbh[1] += d1;
         dbh[2] += d2;
         auto put = [&](float v, int c) {
-          const _Float16 hi = (_Float16)v;
-          const _Float16 lo = (_Float16)(v - (float)hi);
-          s.dy[0][r][c] = __builtin_bit_cast(uint16_t, hi);
-          s.dy[1][r][c] = __builtin_bit_cast(uint16_t, lo);
+#pragma unroll
+          for (int n = 0; n < 3; ++n) {
+            const __bf16 p = (__bf16)v;
+            s.dy[n][r][c] = __builtin_bit_cast(uint16_t, p);
+            v -= (float)p;
+          }
         };
-        put(d0 * sy[0], lane);
-        put(d1 * sy[1], 64 + lane);
-        put(d2 * sy[2], 128 + lane);
+        put(d0, lane);
+        put(d1, 64 + lane);
+        put(d2, 128 + lane);
       }
     }
     __syncthreads();
 
     // ---- dh2 = Wh^T dhy (features 16w .. of both row tiles); dWh += dhy^T h2
     {
-      floatx4 c[2] = {{0.0f, 0.0f, 0.0f, 0.0f}, {0.0f, 0.0f, 0.0f, 0.0f}};
+      floatx4 c[2][2] = {};                     // [row tile][leading | others]
 #pragma unroll
-      for (int h = 0; h < 3; ++h) {              // K steps 2h, 2h + 1: head h's units
-        floatx4 u[2] = {{0.0f, 0.0f, 0.0f, 0.0f}, {0.0f, 0.0f, 0.0f, 0.0f}};
+      for (int k = 0; k < 6; ++k)
 #pragma unroll
-        for (int k = 2 * h; k < 2 * h + 2; ++k)
-#pragma unroll
-          for (int rt = 0; rt < 2; ++rt) {
-            const int at = 32 * k + 8 * q;
-            u[rt] = mfma4(wd[k][0], wd[k][1], ld8(&s.dy[0][16 * rt + r16][at]),
-                          ld8(&s.dy[1][16 * rt + r16][at]), u[rt]);
-          }
-        const float inv = uniform(1.0f / (swh * sy[h]));
-#pragma unroll
-        for (int rt = 0; rt < 2; ++rt) c[rt] += u[rt] * inv;
-      }
+        for (int rt = 0; rt < 2; ++rt) mfma6(wd[k], ld_pieces(s.dy, 16 * rt + r16, 32 * k + 8 * q).p, c[rt]);
 #pragma unroll
       for (int rt = 0; rt < 2; ++rt)
-        *reinterpret_cast<floatx4*>(&s.ex[16 * rt + r16][16 * w + 4 * q]) = c[rt];
-      half8 ah[3], al[3];
+        *reinterpret_cast<floatx4*>(&s.ex[16 * rt + r16][16 * w + 4 * q]) = c[rt][1] + c[rt][0];
+      bf8 av[3][3];
 #pragma unroll
-      for (int i = 0; i < 3; ++i) {
-        ah[i] = ld_rows<YS>(&s.dy[0][0][0], 3 * ta + i, lane);
-        al[i] = ld_rows<YS>(&s.dy[1][0][0], 3 * ta + i, lane);
-      }
+      for (int i = 0; i < 3; ++i)
+#pragma unroll
+        for (int n = 0; n < 3; ++n) av[i][n] = ld_rows(s.dy[n], 3 * ta + i, lane);
 #pragma unroll
       for (int n = 0; n < 4; ++n) {
-        const half8 bh = ld_rows<HS>(&s.h2[0][0][0], 4 * tb + n, lane);
-        const half8 bl = ld_rows<HS>(&s.h2[1][0][0], 4 * tb + n, lane);
+        bf8 b[3];
 #pragma unroll
-        for (int i = 0; i < 3; ++i) dwh[i][n] = mfma3(ah[i], al[i], bh, bl, dwh[i][n]);
+        for (int m = 0; m < 3; ++m) b[m] = ld_rows(s.h2[m], 4 * tb + n, lane);
+#pragma unroll
+        for (int i = 0; i < 3; ++i) dwh[i][n] = mfma6(av[i], b, dwh[i][n]);
         if (n & 1) __builtin_amdgcn_sched_barrier(0);
       }
     }
@@ -697,68 +638,37 @@ __global__ __launch_bounds__(T) void ppo_step_kernel(const qqt_ppo_step_args a, 
     float dv[8], tg[8], tb8[8];
     load8(&s.ex[row][8 * j], dv);
     ln_backward(dv, x2, s.ln[2] + 8 * j, s.ln[3] + 8 * j, rs2, tg, tb8);
-    {
-      float m = 0.0f;
-#pragma unroll
-      for (int i = 0; i < 8; ++i) m = fmaxf(m, fabsf(dv[i]));
-      m = max64(m);
-      if (lane == 0) s.zred[w] = m;
-    }
+    put8(dv, s.dz, row, 8 * j);           // (dhy's planes: read before the barrier above)
     add_rows(tg, g2);
     add_rows(tb8, be2);
     add_rows(dv, db1);
-    half8 wu[4][2];
+    bf8 wu[4][3];
 #pragma unroll
-    for (int k = 0; k < 4; ++k)
-#pragma unroll
-      for (int p = 0; p < 2; ++p) wu[k][p] = frag(F_DH1, 4, w, k, p);
-    __syncthreads();
-    {
-      float m = s.zred[0];
-#pragma unroll
-      for (int i = 1; i < 8; ++i) m = fmaxf(m, s.zred[i]);
-      m = uniform(m);
-      if (m * sz > 0x1p15f) {
-        const float ns = uniform(scale_for(m)), f = uniform(ns / sz);
-        sz = ns;
-#pragma unroll
-        for (int i = 0; i < 2; ++i)
-#pragma unroll
-          for (int n = 0; n < 4; ++n) dw1[i][n] *= f;
-      }
-#pragma unroll
-      for (int i = 0; i < 8; ++i) dv[i] *= sz;
-      split8(dv, &s.dz[0][row][8 * j], &s.dz[1][row][8 * j]);
-    }
+    for (int k = 0; k < 4; ++k) frag(wu[k], F_DH1, 4, w, k);
     __syncthreads();
 
     // ---- dh1 = W1^T dz2; dW1 += dz2^T h1
     {
-      floatx4 c[2] = {{0.0f, 0.0f, 0.0f, 0.0f}, {0.0f, 0.0f, 0.0f, 0.0f}};
+      floatx4 c[2][2] = {};                     // [row tile][leading | others]
 #pragma unroll
       for (int k = 0; k < 4; ++k)
 #pragma unroll
-        for (int rt = 0; rt < 2; ++rt) {
-          const int at = 32 * k + 8 * q;
-          c[rt] = mfma4(wu[k][0], wu[k][1], ld8(&s.dz[0][16 * rt + r16][at]),
-                        ld8(&s.dz[1][16 * rt + r16][at]), c[rt]);
-        }
-      const float inv = uniform(1.0f / (sw1 * sz));
+        for (int rt = 0; rt < 2; ++rt) mfma6(wu[k], ld_pieces(s.dz, 16 * rt + r16, 32 * k + 8 * q).p, c[rt]);
 #pragma unroll
       for (int rt = 0; rt < 2; ++rt)
-        *reinterpret_cast<floatx4*>(&s.ex[16 * rt + r16][16 * w + 4 * q]) = c[rt] * inv;
-      half8 ah[2], al[2];
+        *reinterpret_cast<floatx4*>(&s.ex[16 * rt + r16][16 * w + 4 * q]) = c[rt][1] + c[rt][0];
+      bf8 av[2][3];
 #pragma unroll
-      for (int i = 0; i < 2; ++i) {
-        ah[i] = ld_rows<HS>(&s.dz[0][0][0], 2 * ta + i, lane);
-        al[i] = ld_rows<HS>(&s.dz[1][0][0], 2 * ta + i, lane);
-      }
+      for (int i = 0; i < 2; ++i)
+#pragma unroll
+        for (int n = 0; n < 3; ++n) av[i][n] = ld_rows(s.dz[n], 2 * ta + i, lane);
 #pragma unroll
       for (int n = 0; n < 4; ++n) {
-        const half8 bh = ld_rows<HS>(&s.h1[0][0][0], 4 * tb + n, lane);
-        const half8 bl = ld_rows<HS>(&s.h1[1][0][0], 4 * tb + n, lane);
+        bf8 b[3];
 #pragma unroll
-        for (int i = 0; i < 2; ++i) dw1[i][n] = mfma3(ah[i], al[i], bh, bl, dw1[i][n]);
+        for (int m = 0; m < 3; ++m) b[m] = ld_rows(s.h1[m], 4 * tb + n, lane);
+#pragma unroll
+        for (int i = 0; i < 2; ++i) dw1[i][n] = mfma6(av[i], b, dw1[i][n]);
         if (n & 1) __builtin_amdgcn_sched_barrier(0);
       }
     }
@@ -787,17 +697,15 @@ __global__ __launch_bounds__(T) void ppo_step_kernel(const qqt_ppo_step_args a, 
   // ---- this workgroup's partial sums
   float* const P = reinterpret_cast<float*>(static_cast<char*>(a.workspace) + WS_PART) +
                    (size_t)blockIdx.x * P_PAD;
-  const float iw1 = 1.0f / sz / sh1;
-  const float iwh[3] = {1.0f / sy[0] / sh2, 1.0f / sy[1] / sh2, 1.0f / sy[2] / sh2};
 #pragma unroll
   for (int n = 0; n < 4; ++n)
 #pragma unroll
     for (int i = 0; i < 4; ++i) {
       const int col = 16 * (4 * tb + n) + r16;
 #pragma unroll
-      for (int u = 0; u < 3; ++u) P[P_WH + (16 * (3 * ta + u) + 4 * q + i) * H + col] = dwh[u][n][i] * iwh[(3 * ta + u) >> 2];
+      for (int u = 0; u < 3; ++u) P[P_WH + (16 * (3 * ta + u) + 4 * q + i) * H + col] = dwh[u][n][i];
 #pragma unroll
-      for (int u = 0; u < 2; ++u) P[P_W1 + (16 * (2 * ta + u) + 4 * q + i) * H + col] = dw1[u][n][i] * iw1;
+      for (int u = 0; u < 2; ++u) P[P_W1 + (16 * (2 * ta + u) + 4 * q + i) * H + col] = dw1[u][n][i];
     }
   // per-wavefront sums meet in LDS: columns (6 kinds), output layer, biases
   float* const cs = &s.hy[0][0];                 // [8 wavefronts][6][128] = 24.6 KB
@@ -819,6 +727,8 @@ __global__ __launch_bounds__(T) void ppo_step_kernel(const qqt_ppo_step_args a, 
     for (int k = 0; k < 8; ++k) fs[(w * 8 + k) * 64 + lane] = dwf[k];
 #pragma unroll
     for (int k = 0; k < 3; ++k) hs[w * HY + 64 * k + lane] = dbh[k];
+    const float m = max64(s.sum[2][row][j]);
+    if (lane == 0) s.mx[w] = m;
   }
   __syncthreads();
   for (int i = t; i < 6 * H; i += T) {
@@ -838,17 +748,18 @@ __global__ __launch_bounds__(T) void ppo_step_kernel(const qqt_ppo_step_args a, 
 #pragma unroll
     for (int k = 0; k < 8; ++k) u[k] = hs[k * HY + t];
     P[P_DBH + t] = tree8(u);
-  } else if (t < HY + 8) {
-    float v = 0.0f;
-    for (int r = 0; r < R; ++r) v += s.sum[0][r][2 * (t - HY)];
-    P[P_DBF + t - HY] = v;
-  } else if (t < HY + 13) {
-    float v = 0.0f;
-    for (int r = 0; r < R; ++r) v += s.sum[1][r][t - HY - 8];
-    P[P_ST + t - HY - 8] = v;
+  } else if (t < HY + 13) {                            // output biases, statistics
+    const int k = t - HY;
+    const float(*const rows)[16] = k < 8 ? s.sum[0] : s.sum[1];
+    const int c = k < 8 ? 2 * k : k - 8;
+    float u[8];
+#pragma unroll
+    for (int n = 0; n < 8; ++n)
+      u[n] = (rows[4 * n][c] + rows[4 * n + 1][c]) + (rows[4 * n + 2][c] + rows[4 * n + 3][c]);
+    P[P_DBF + k] = tree8(u);                            // DBF, ST in order
   } else if (t == HY + 13) {
     float v = 0.0f;
-    for (int r = 0; r < R * 16; ++r) v = fmaxf(v, s.sum[2][0][r]);
+    for (int k = 0; k < 8; ++k) v = fmaxf(v, s.mx[k]);
     P[P_MX] = v;
   }
 }

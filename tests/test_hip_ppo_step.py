@@ -86,6 +86,126 @@ def test_gradients_against_float64(b, outliers):
     assert bool(torch.isfinite(dw0).all()) and float(dw0.abs().max()) > 0.0
 
 
+def _row_losses(w, z1, mm, bm, act, old_logp, adv, ret, old_val, cfg, entropy_coef):
+    """Each row's loss in float64 and how far it is from the nearest kink (a
+    ReLU input at zero, a ratio or value at its clip bound, a tie of the two
+    value errors)."""
+    ln = torch.nn.functional.layer_norm
+    a1 = ln(z1, (128,), w["shared.1.weight"], w["shared.1.bias"])
+    a2 = ln(torch.relu(a1) @ w["shared.3.weight"].t() + w["shared.3.bias"], (128,),
+            w["shared.4.weight"], w["shared.4.bias"])
+    near, o = [a1, a2], []
+    for h in ("move_head", "bomb_head", "critic"):
+        near.append(torch.relu(a2) @ w[f"{h}.0.weight"].t() + w[f"{h}.0.bias"])
+        o.append(torch.relu(near[-1]) @ w[f"{h}.2.weight"].t() + w[f"{h}.2.bias"])
+    logp, ent = 0.0, 0.0
+    for lg, mask, a in ((o[0], mm, act[:, 0]), (o[1], bm, act[:, 1])):
+        ls = torch.log_softmax(lg.masked_fill(~mask, torch.finfo(torch.float32).min), -1)
+        logp = logp + ls.gather(-1, a[:, None])[:, 0]
+        ent = ent - (ls.exp() * ls).sum(-1)
+    v, e = o[2][:, 0], cfg.clip_eps
+    ratio, dv = (logp - old_logp.double()).exp(), v - old_val
+    vc = old_val + dv.clamp(-e, e)
+    loss = (-torch.min(ratio * adv, ratio.clamp(1 - e, 1 + e) * adv) - entropy_coef * ent
+            + 0.5 * cfg.value_coef * torch.maximum((v - ret) ** 2, (vc - ret) ** 2))
+    tie = torch.where(vc == v, torch.ones_like(v), ((v - ret).abs() - (vc - ret).abs()).abs())
+    near = [torch.cat(near, 1).abs().amin(1), (ratio - 1 - e).abs(), (ratio - 1 + e).abs(),
+            (dv.abs() - e).abs(), tie]
+    return loss, torch.stack(near).amin(0)
+
+
+def _smooth_rows(net, b, seed, dev, cfg, entropy_coef, scale_rows):
+    """b rows of `_case` none of which is within rounding of a kink (there a
+    correct float32 result may take either branch), their z1 and weights."""
+    args = _case(b + b // 8 + 64, seed, dev, False)
+    old_logp, adv, ret, old_val = args[4:]
+    scale_rows(adv, ret, old_val)
+    lin = net.shared[0]
+    w = {k: v.detach().double() for k, v in net.named_parameters()}
+    with torch.no_grad():
+        z1 = net._l1_forward(args[0], lin.weight, lin.bias, 0)
+        near = _row_losses(w, z1.double(), *args[1:], cfg, entropy_coef)[1]
+        keep = (near > 3e-6).nonzero()[:, 0][:b]
+        assert keep.numel() == b
+        args = tuple(x[keep].contiguous() for x in args)
+        return args, net._l1_forward(args[0], lin.weight, lin.bias, 0), w
+
+
+def _spread_net(seed, dev):
+    from qqtsim import HipMlpActorCritic, reference_init
+
+    sd = reference_init(seed=seed)
+    g = torch.Generator().manual_seed(seed)
+    for k in sd:
+        if k.endswith("2.weight"):
+            sd[k] = sd[k] + 0.1 * torch.randn(sd[k].shape, generator=g)
+    return HipMlpActorCritic(device=dev, state_dict=sd)
+
+
+@pytest.mark.gpu
+def test_rows_do_not_share_precision():
+    """dz1 of every row against float64, with row gradients of one batch spread
+    over nine orders of magnitude in random order (40,001 rows: four and five
+    tiles per workgroup): a row beside or behind a larger one keeps float32's
+    bits.  Bound: sums of up to 192 float32 products through three layers and
+    two LayerNorm backwards (differences of like terms) are about 2^-22 of the
+    row's norm, some four times that (1e-6) for the worst of 40,001 rows, and as
+    much again for another order of the sums: 4e-6."""
+    from qqtsim import PPOConfig
+
+    dev, cfg, b = torch.device("cuda:0"), PPOConfig(value_coef=0.0), 40_001
+    net = _spread_net(21, dev)
+
+    def scale_rows(adv, ret, old_val):   # (policy term alone: a value error is v's own rounding)
+        size = 10.0 ** (-9.0 * torch.rand(adv.shape, generator=torch.Generator().manual_seed(2)))
+        adv *= size.to(dev)
+
+    args, z1, w = _smooth_rows(net, b, 21, dev, cfg, 0.0, scale_rows)
+    got = {}
+    inner = net._l1_weight_grad
+    net._l1_weight_grad = lambda x, dz1, *a, **k: got.update(dz1=dz1.clone()) or inner(x, dz1, *a, **k)
+    net.ppo_grads(*args, cfg, 0.0)
+    x = z1.double().requires_grad_(True)
+    (_row_losses(w, x, *args[1:], cfg, 0.0)[0].sum() / b).backward()
+    # (rows that the clip or a single legal action leaves without a gradient drop out)
+    rows = x.grad.norm(dim=1) > 1e-3 * args[5].abs().double() / b
+    assert int(rows.sum()) > b // 4
+    err = (got["dz1"].double() - x.grad).norm(dim=1)[rows] / x.grad.norm(dim=1)[rows]
+    print(f"worst row {float(err.max()):.2e}, median {float(err.median()):.2e}")
+    assert float(err.max()) <= 4e-6
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("b", [8193, 40_001])
+def test_gradients_of_several_tiles_against_float64(b):
+    """Two to five tiles per workgroup, with policy and value outliers of 30
+    and 100 times the others in second and later tiles (the earlier tiles still
+    matter in every sum), rows within rounding of a kink left out.  Bound: 8
+    times the 1.2e-7 that float32 sums of these products show."""
+    from qqtsim import PPOConfig
+
+    dev, cfg = torch.device("cuda:0"), PPOConfig()
+    net = _spread_net(b, dev)
+
+    def scale_rows(adv, ret, old_val):
+        late = torch.arange(8192, adv.numel(), 37, device=dev)
+        adv[late[::2]] *= 30.0
+        ret[late[1::2]] *= 100.0
+
+    args, z1, w = _smooth_rows(net, b, b, dev, cfg, 0.05, scale_rows)
+    net.ppo_grads(*args, cfg, 0.05)
+    for v in w.values():
+        v.requires_grad_(True)
+    x = z1.double() + (w["shared.0.bias"] - w["shared.0.bias"].detach())
+    loss, _ = _row_losses(w, x, *args[1:], cfg, 0.05)
+    (loss.sum() / b).backward()
+    for k, p in net.named_parameters():
+        if k != "shared.0.weight":
+            err = float((p.grad.double() - w[k].grad).norm() / w[k].grad.norm())
+            print(f"{k} {err:.2e}")
+            assert err <= 1e-6, (k, err)
+
+
 @pytest.mark.gpu
 def test_parameters_that_view_a_flat_buffer():
     """Parameters at any element of one flat buffer (not 16-byte aligned) are
