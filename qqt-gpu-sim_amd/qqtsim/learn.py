@@ -102,13 +102,24 @@ class _Linear(torch.autograd.Function):
         return dy @ w, _weight_grad(dy, x), dy.sum(0)
 
 
+def _seq_weight_grad(dy: torch.Tensor, x: torch.Tensor) -> torch.Tensor:
+    """`_weight_grad` for the recurrence's weights: chunks short enough that a
+    float32 sum within one is no longer than a frame's own product would be
+    (error against float64 of dW_ih and dW_hh, 32 frames x 256 envs: chunks of
+    256 rows 1.8e-7, of 1,024 2.6e-7, of 4,096 7.4e-7, frame by frame through
+    nn.LSTM 2.0e-7; 12 x 37: chunks of 64 6.0e-7, of 256 1.0e-6, nn.LSTM
+    6.2e-7), and at most a few hundred of them."""
+    return _weight_grad(dy, x, chunk=min(512, max(64, dy.shape[0] // 32)))
+
+
 class _InputProduct(_Linear):
     """The same product for the recurrence's inputs, summed over quarters of
     the reduction: one sum over all 256 inputs leaves an error in the gates
     that is larger than everything the recurrence adds (hidden outputs of 32
     frames x 256 envs against float64, mean of eight inputs: 1.37e-7 relative
     with one sum, 1.05e-7 with quarters, 1.06e-7 through nn.LSTM's own
-    kernels)."""
+    kernels).  The input gradient sums eighths of its 512 gates: 12 x 37 frames 2.4e-7 in
+    quarters, 1.8e-7 through nn.LSTM."""
 
     @staticmethod
     def forward(ctx, x, w, b):
@@ -119,6 +130,16 @@ class _InputProduct(_Linear):
         for p in parts[1:]:
             out.addmm_(*p)
         return out
+
+    @staticmethod
+    def backward(ctx, dy):
+        x, w = ctx.saved_tensors
+        dy = dy.contiguous()
+        step = -(-w.shape[0] // 8)
+        dx = dy[:, :step] @ w[:step]
+        for k in range(step, w.shape[0], step):
+            dx = torch.addmm(dx, dy[:, k:k + step], w[k:k + step])
+        return dx, _seq_weight_grad(dy, x), dy.sum(0)
 
 
 def _lin(mod: nn.Linear, x):
@@ -530,7 +551,7 @@ class _Recurrence(torch.autograd.Function):
         if ctx.needs_input_grad[1]:
             if keep.shape[0] > 1:
                 before = (h[:-1] * keep[:-1].unsqueeze(-1)).view(-1, HID)
-                dw = _weight_grad(dz[1:].view(-1, 4 * HID), before, chunk=1024)
+                dw = _seq_weight_grad(dz[1:].view(-1, 4 * HID), before)
             else:
                 dw = torch.zeros_like(w_hh)
         return dz if ctx.needs_input_grad[0] else None, dw, None, None

@@ -60,6 +60,45 @@ def test_sequence_kernels_match_the_frame_by_frame_recurrence(steps, m, window):
         assert rel(p.grad, q.grad) < 5e-6, k
 
 
+@pytest.mark.gpu
+@pytest.mark.parametrize("steps,m", [(12, 37), (32, 256), (24, 1400)])
+def test_weight_gradients_keep_the_precision_of_frame_products(steps, m):
+    """dW_ih, dW_hh and the input gradient are no further from float64 than
+    nn.LSTM called frame by frame is (the update's path for modules that the
+    sequence kernels do not serve).  Bound: 1.25 times its error, for sums in
+    another order; one sum over 4,096 rows is at four times."""
+    from qqtsim.learn import _sequence_outputs
+
+    torch.manual_seed(steps + m)
+    lstm = torch.nn.LSTM(256, HID, batch_first=True).cuda()
+    base = torch.randn(steps, m, 256, device="cuda").relu()
+    keep = (torch.rand(steps, m, device="cuda") > 0.05).float()
+    dy = torch.randn(steps, m, HID, device="cuda")
+
+    def by_module(x, net):
+        state, outs = None, []
+        for t in range(steps):
+            out, state = net(x[t].unsqueeze(1), state)
+            outs.append(out.squeeze(1))
+            state = tuple(v * keep[t][:, None].to(v.dtype) for v in state)
+        return torch.stack(outs)
+
+    def grads(run, dtype):
+        net = torch.nn.LSTM(256, HID, batch_first=True).cuda().to(dtype)
+        net.load_state_dict({k: v.to(dtype) for k, v in lstm.state_dict().items()})
+        x = base.to(dtype).clone().requires_grad_(True)
+        run(x, net).backward(dy.to(dtype))
+        return dict(ih=net.weight_ih_l0.grad, hh=net.weight_hh_l0.grad, x=x.grad)
+
+    want = grads(lambda x, net: _frame_by_frame(x, net, keep.double(), 0), torch.float64)
+    got = grads(lambda x, net: _sequence_outputs(net, x, keep, 0), torch.float32)
+    module = grads(by_module, torch.float32)
+    for k, w in want.items():
+        mine, theirs = (float((g[k].double() - w).norm() / w.norm()) for g in (got, module))
+        print(f"{k}: {mine:.2e}, frame by frame {theirs:.2e}")
+        assert mine <= 1.25 * theirs, k
+
+
 def test_only_a_plain_float32_lstm_on_the_gpu_is_served():
     from qqtsim.learn import _sequence_kernels_serve
 
