@@ -514,6 +514,13 @@ def _masked_logp_entropy(ml, bl, mm, bm, act):
     return logp, ent
 
 
+def _aligned(t: torch.Tensor) -> torch.Tensor:
+    """t, contiguous and on 16 bytes (a view into a flat buffer, a parameter or
+    one that a saved-tensor hook returns, may lie at any element)."""
+    t = t.contiguous()
+    return t.clone() if t.data_ptr() % 16 else t
+
+
 class _Recurrence(torch.autograd.Function):
     """(T, m, 128) hidden outputs of the recurrence z = zx + h W_hh^T over T
     frames from the zero state, the state multiplied by keep[t] after frame t
@@ -540,7 +547,8 @@ class _Recurrence(torch.autograd.Function):
     @torch.autograd.function.once_differentiable
     def backward(ctx, dh):
         w_hh, keep, h, c, gates = ctx.saved_tensors
-        w_hh, keep, h, c, gates, dh = (t.contiguous() for t in (w_hh, keep, h, c, gates, dh))
+        w_hh = _aligned(w_hh)
+        keep, h, c, gates, dh = (t.contiguous() for t in (keep, h, c, gates, dh))
         dz = torch.empty_like(gates)
         a = _capi.LstmSeqArgsC()
         a.steps, a.rows, a.window = *keep.shape, ctx.window
@@ -586,10 +594,8 @@ def _sequence_outputs(lstm, fused, keep, window: int):
     steps, m, width = fused.shape
     zx = _InputProduct.apply(fused.reshape(steps * m, width), lstm.weight_ih_l0,
                        lstm.bias_ih_l0 + lstm.bias_hh_l0)
-    w_hh = lstm.weight_hh_l0.contiguous()
-    if w_hh.data_ptr() % 16:
-        w_hh = w_hh.clone()
-    return _Recurrence.apply(zx.view(steps, m, -1).contiguous(), w_hh, keep.contiguous(), window)
+    return _Recurrence.apply(zx.view(steps, m, -1).contiguous(), _aligned(lstm.weight_hh_l0),
+                             keep.contiguous(), window)
 
 
 def _lstm_update(learner, opt, buf, last_val, cfg: PPOConfig, entropy_coef: float) -> dict:

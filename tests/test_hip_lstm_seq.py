@@ -99,6 +99,35 @@ def test_weight_gradients_keep_the_precision_of_frame_products(steps, m):
         assert mine <= 1.25 * theirs, k
 
 
+@pytest.mark.gpu
+def test_weights_and_saved_tensors_at_any_element():
+    """W_hh as a view into a flat buffer, and tensors that a saved-tensor hook
+    hands back at an odd element: the gradients of the plain call."""
+    from qqtsim.learn import _sequence_outputs
+
+    torch.manual_seed(5)
+    steps, m = 5, 19
+    x = torch.randn(steps, m, 256, device="cuda")
+    keep = (torch.rand(steps, m, device="cuda") > 0.2).float()
+    dy = torch.randn(steps, m, HID, device="cuda")
+    plain = torch.nn.LSTM(256, HID, batch_first=True).cuda()
+    moved = torch.nn.LSTM(256, HID, batch_first=True).cuda()
+    for k in ("weight_ih_l0", "weight_hh_l0", "bias_ih_l0", "bias_hh_l0"):
+        p = getattr(plain, k).detach()
+        view = torch.zeros(p.numel() + 1, device="cuda")[1:].view(p.shape)
+        getattr(moved, k).data = view.copy_(p)
+    assert moved.weight_hh_l0.data_ptr() % 16
+
+    def pack(t):
+        return torch.cat([t.new_zeros(1), t.detach().reshape(-1)]), t.shape
+
+    _sequence_outputs(plain, x, keep, 2).backward(dy)
+    with torch.autograd.graph.saved_tensors_hooks(pack, lambda s: s[0][1:].view(s[1])):
+        _sequence_outputs(moved, x, keep, 2).backward(dy)
+    for (k, p), (_, q) in zip(plain.named_parameters(), moved.named_parameters()):
+        assert torch.equal(p.grad, q.grad), k
+
+
 def test_only_a_plain_float32_lstm_on_the_gpu_is_served():
     from qqtsim.learn import _sequence_kernels_serve
 
