@@ -72,6 +72,33 @@ def test_lstm_update_matches_the_reference_restatement(dev):
     assert moved > 1e-4 and worst <= 2e-6
 
 
+def test_a_hooked_lstm_is_called_frame_by_frame(dev):
+    """A module with a hook is called for every frame (the sequence kernels
+    would pass it by), and the update is the same against the restatement."""
+    from oracle.ppo_lstm import lstm_update
+    from qqtsim import LstmLearner, PPOConfig, ppo_update
+
+    n, T, seed = 48, 14, 6
+    sim, net, roll, buf = _collect(dev, n, T, seed)
+    last_val = roll.last_value()
+    cfg = PPOConfig(epochs=2, minibatches=3, bptt_window=5)
+    a = LstmLearner().to(dev)
+    b = copy.deepcopy(a)
+    calls = []
+    a.lstm.register_forward_hook(lambda *_: calls.append(1))
+    oa = torch.optim.SGD(a.parameters(), lr=0.05)
+    ob = torch.optim.SGD(b.parameters(), lr=0.05)
+    torch.manual_seed(3)
+    got = ppo_update(a, oa, buf, last_val, cfg, 0.05)
+    torch.manual_seed(3)
+    want = lstm_update(b, ob, buf, last_val, cfg, 0.05)
+    assert len(calls) == 2 * 3 * T
+    for k in want:
+        assert abs(got[k] - want[k]) <= 1e-5 * max(1.0, abs(want[k])), k
+    for (name, pa), (_, pb) in zip(a.named_parameters(), b.named_parameters()):
+        assert float((pa - pb).detach().abs().max()) <= 2e-6, name
+
+
 def test_lstm_training_iterations_stay_finite_and_sync(dev):
     """Two collect + update iterations with Adam and the weight sync to the
     acting network; after the sync the acting kernel reproduces the
