@@ -217,10 +217,10 @@ def test_ppo_update_runs_on_a_collected_buffer(dev):
 
 
 def test_fused_ppo_grads_match_autograd(dev):
-    """qqt_ppo_grad (+ the first layer's kernels): every parameter gradient
+    """ppo_grads (qqt_ppo_step and the first layer's kernels): every parameter gradient
     and the five statistics equal what loss.backward() through evaluate()
     gives on the same module (float32, summation order aside), on a ragged
-    batch (3001 rows: the last 16-row block is partial) with masked moves,
+    batch (3001 rows: the last 32-row tile is partial) with masked moves,
     masked bombs, clipped and unclipped ratios and value errors."""
     from qqtsim.learn import HipMlpActorCritic, PPOConfig
 
