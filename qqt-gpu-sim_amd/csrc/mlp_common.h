@@ -30,6 +30,22 @@ constexpr int W1_HALVES = HID * HID;         // one plane of the layer-2 fragmen
 constexpr int WH_HALVES = 3 * HEAD * HID;    // one plane of the head-layer fragments (48 KB)
 constexpr int WF_HALVES = 16 * 3 * HEAD;     // one plane of the output-layer fragments (6 KB)
 
+typedef short s4 __attribute__((ext_vector_type(4)));
+typedef __attribute__((address_space(3))) s4 lds_s4;
+
+// Transposed operand (V: eight 16-bit values) of a contraction over 32 LDS
+// rows of S values: element i of lane (r16, q) is row 8q + i, column 16 tile +
+// r16.  Two transposing reads: lanes 4a..4a+3 of a 16-lane group address row
+// 8q + a (32 bytes), and lane j receives column j of those four rows.
+template <class V, int S>
+__device__ __forceinline__ V ld_rows(const uint16_t* plane, int tile, int lane) {
+  const int q = lane >> 4, j = lane & 15;
+  const uint16_t* p = plane + (8 * q + (j >> 2)) * S + 16 * tile + 4 * (j & 3);
+  const s4 a = __builtin_amdgcn_ds_read_tr16_b64_v4i16((lds_s4*)(p));
+  const s4 b = __builtin_amdgcn_ds_read_tr16_b64_v4i16((lds_s4*)(p + 4 * S));
+  return __builtin_bit_cast(V, __builtin_shufflevector(a, b, 0, 1, 2, 3, 4, 5, 6, 7));
+}
+
 struct Frag16 { half8 lo, hi; };   // 16 halves of one lane in one K block
 
 __device__ __forceinline__ half8 as_h8(uint4 v) {

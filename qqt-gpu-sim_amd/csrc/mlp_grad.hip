@@ -40,6 +40,7 @@
 #include <mutex>
 #include <type_traits>
 
+#include "mlp_common.h"
 #include "qqt_common.h"
 #include "qqt_hip.h"
 #include "qqt_learn.h"
@@ -50,10 +51,6 @@ extern thread_local char g_err[512];
 
 namespace l1g {
 
-typedef _Float16 half8 __attribute__((ext_vector_type(8)));
-typedef float floatx4 __attribute__((ext_vector_type(4)));
-
-constexpr int HID = 128;          // first-layer outputs
 constexpr int NCOL = 512;         // observation columns per workgroup ...
 constexpr int NARROW = 128;       // ... and where its slot takes several chunks or the grid is small
 constexpr int KS = 32;            // batch rows per step (one MFMA K)
@@ -67,31 +64,11 @@ constexpr int TARGET_WGS = 256;   // one workgroup (104 KB of LDS, 256 registers
 constexpr int CHUNK_ROWS = 512;   // least rows of a chunk
 constexpr int SLOT_ROWS = 2048;   // ... of a slot of the workspace every caller provides
 
-typedef short s4 __attribute__((ext_vector_type(4)));
-typedef __attribute__((address_space(3))) s4 lds_s4;
-typedef uint32_t u32x4 __attribute__((ext_vector_type(4)));
-
-__device__ __forceinline__ floatx4 mfma(half8 a, half8 b, floatx4 c) {
-  return __builtin_amdgcn_mfma_f32_16x16x32_f16(a, b, c, 0, 0, 0);
-}
-
 template <int NC>
 struct __align__(16) Lds {
   uint16_t x[2][KS][NC + 16];     // observation rows
   uint16_t d[2][2][KS][DS];       // dz1 rows, hi and lo planes
 };
-
-// Element i of lane (r16, q): row 8q + i, column 16 tile + r16 of an LDS plane
-// with row stride S: lanes 4a..4a+3 of a 16-lane group address row 8q + a
-// (32 bytes) and lane j receives column j of those four rows.
-template <int S>
-__device__ __forceinline__ half8 ld_rows(const uint16_t* plane, int tile, int lane) {
-  const int q = lane >> 4, j = lane & 15;
-  const uint16_t* p = plane + (8 * q + (j >> 2)) * S + 16 * tile + 4 * (j & 3);
-  const s4 a = __builtin_amdgcn_ds_read_tr16_b64_v4i16((lds_s4*)(p));
-  const s4 b = __builtin_amdgcn_ds_read_tr16_b64_v4i16((lds_s4*)(p + 4 * S));
-  return __builtin_bit_cast(half8, __builtin_shufflevector(a, b, 0, 1, 2, 3, 4, 5, 6, 7));
-}
 
 // Accumulators of a wavefront: four m tiles x JT n tiles.
 template <int NC>
@@ -196,11 +173,11 @@ __device__ __forceinline__ void l1_grad_chunk(const qqt_l1_grad_args& a, Lds<NC>
     if constexpr (NC == NARROW) {       // few n tiles: hold those, pass the m tiles through
       half8 b[JT];
 #pragma unroll
-      for (int j = 0; j < JT; ++j) b[j] = ld_rows<XS>(&s.x[buf][0][0], nt + j, lane);
+      for (int j = 0; j < JT; ++j) b[j] = ld_rows<half8, XS>(&s.x[buf][0][0], nt + j, lane);
 #pragma unroll
       for (int i = 0; i < 4; ++i) {
-        const half8 ah = ld_rows<DS>(&s.d[buf][0][0][0], mt + i, lane);
-        const half8 al = ld_rows<DS>(&s.d[buf][1][0][0], mt + i, lane);
+        const half8 ah = ld_rows<half8, DS>(&s.d[buf][0][0][0], mt + i, lane);
+        const half8 al = ld_rows<half8, DS>(&s.d[buf][1][0][0], mt + i, lane);
 #pragma unroll
         for (int j = 0; j < JT; ++j) acc.v[i][j] = mfma(ah, b[j], acc.v[i][j]);
 #pragma unroll
@@ -210,12 +187,12 @@ __device__ __forceinline__ void l1_grad_chunk(const qqt_l1_grad_args& a, Lds<NC>
       half8 ah[4], al[4];
 #pragma unroll
       for (int i = 0; i < 4; ++i) {
-        ah[i] = ld_rows<DS>(&s.d[buf][0][0][0], mt + i, lane);
-        al[i] = ld_rows<DS>(&s.d[buf][1][0][0], mt + i, lane);
+        ah[i] = ld_rows<half8, DS>(&s.d[buf][0][0][0], mt + i, lane);
+        al[i] = ld_rows<half8, DS>(&s.d[buf][1][0][0], mt + i, lane);
       }
 #pragma unroll
       for (int j = 0; j < JT; ++j) {
-        const half8 b = ld_rows<XS>(&s.x[buf][0][0], nt + j, lane);
+        const half8 b = ld_rows<half8, XS>(&s.x[buf][0][0], nt + j, lane);
 #pragma unroll
         for (int i = 0; i < 4; ++i) acc.v[i][j] = mfma(ah[i], b, acc.v[i][j]);
 #pragma unroll
@@ -425,7 +402,7 @@ __host__ inline int64_t slot_floats(int k0) {
 // to a kernel (on the host it is only a stand-in for the symbol): it uses
 // the device address hipGetSymbolAddress returns for the current device.
 static __device__ __align__(256) float
-    l1g_scratch[l1g::MAX_CHUNKS * l1g::HID * QQT_L1_GRAD_NOALLOC_MAX_K0];
+    l1g_scratch[l1g::MAX_CHUNKS * HID * QQT_L1_GRAD_NOALLOC_MAX_K0];
 
 namespace l1g {
 
@@ -607,7 +584,7 @@ int qqt_l1_grad_noalloc(const qqt_l1_grad_args* a, void* stream) {
   qqt_l1_grad_args b = *a;          // the caller's workspace fields are ignored
   b.workspace = ptr;
   b.workspace_floats = qqt_l1_grad_preferred_floats(b.batch, b.k0);
-  if (b.workspace_floats > (int64_t)l1g::MAX_CHUNKS * l1g::HID * QQT_L1_GRAD_NOALLOC_MAX_K0) {
+  if (b.workspace_floats > (int64_t)l1g::MAX_CHUNKS * HID * QQT_L1_GRAD_NOALLOC_MAX_K0) {
     snprintf(g_err, sizeof(g_err), "qqt_l1_grad_noalloc: plan exceeds the static scratch");
     return QQT_E_ARG;
   }

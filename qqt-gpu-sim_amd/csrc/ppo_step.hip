@@ -96,8 +96,6 @@ constexpr size_t WS_PART = (size_t)F_END * 2;
 
 typedef __bf16 bf8 __attribute__((ext_vector_type(8)));
 typedef float float8v __attribute__((ext_vector_type(8)));
-typedef short s4 __attribute__((ext_vector_type(4)));
-typedef __attribute__((address_space(3))) s4 lds_s4;
 
 struct __align__(16) Lds {
   uint16_t h1[3][R][HS], h2[3][R][HS];      // pieces of h1, h2
@@ -171,19 +169,6 @@ __device__ __forceinline__ void put8(const float (&v)[8], uint16_t (&plane)[3][R
   split8(v, p);
 #pragma unroll
   for (int k = 0; k < 3; ++k) *reinterpret_cast<bf8*>(&plane[k][row][at]) = p[k];
-}
-
-// Transposed operand of a contraction over the tile's rows: element i of lane
-// (r16, q) is row 8q + i, feature 16 tile + r16 of an LDS plane with row
-// stride S.  One transposing read: lanes 4a..4a+3 of a 16-lane group address
-// row 8q + a (32 bytes), and lane j receives column j of those four rows.
-template <int S>
-__device__ __forceinline__ bf8 ld_rows(const uint16_t (&plane)[R][S], int tile, int lane) {
-  const int q = lane >> 4, j = lane & 15;
-  const uint16_t* p = &plane[8 * q + (j >> 2)][16 * tile + 4 * (j & 3)];
-  const s4 a = __builtin_amdgcn_ds_read_tr16_b64_v4i16((lds_s4*)(p));
-  const s4 b = __builtin_amdgcn_ds_read_tr16_b64_v4i16((lds_s4*)(p + 4 * S));
-  return __builtin_bit_cast(bf8, __builtin_shufflevector(a, b, 0, 1, 2, 3, 4, 5, 6, 7));
 }
 
 // c += a b without the three products below 2^-25 of it
@@ -620,12 +605,12 @@ __global__ __launch_bounds__(T) void ppo_step_kernel(const qqt_ppo_step_args a, 
 #pragma unroll
       for (int i = 0; i < 3; ++i)
 #pragma unroll
-        for (int n = 0; n < 3; ++n) av[i][n] = ld_rows(s.dy[n], 3 * ta + i, lane);
+        for (int n = 0; n < 3; ++n) av[i][n] = ld_rows<bf8, YS>(s.dy[n][0], 3 * ta + i, lane);
 #pragma unroll
       for (int n = 0; n < 4; ++n) {
         bf8 b[3];
 #pragma unroll
-        for (int m = 0; m < 3; ++m) b[m] = ld_rows(s.h2[m], 4 * tb + n, lane);
+        for (int m = 0; m < 3; ++m) b[m] = ld_rows<bf8, HS>(s.h2[m][0], 4 * tb + n, lane);
 #pragma unroll
         for (int i = 0; i < 3; ++i) dwh[i][n] = mfma6(av[i], b, dwh[i][n]);
         if (n & 1) __builtin_amdgcn_sched_barrier(0);
@@ -661,12 +646,12 @@ __global__ __launch_bounds__(T) void ppo_step_kernel(const qqt_ppo_step_args a, 
 #pragma unroll
       for (int i = 0; i < 2; ++i)
 #pragma unroll
-        for (int n = 0; n < 3; ++n) av[i][n] = ld_rows(s.dz[n], 2 * ta + i, lane);
+        for (int n = 0; n < 3; ++n) av[i][n] = ld_rows<bf8, HS>(s.dz[n][0], 2 * ta + i, lane);
 #pragma unroll
       for (int n = 0; n < 4; ++n) {
         bf8 b[3];
 #pragma unroll
-        for (int m = 0; m < 3; ++m) b[m] = ld_rows(s.h1[m], 4 * tb + n, lane);
+        for (int m = 0; m < 3; ++m) b[m] = ld_rows<bf8, HS>(s.h1[m][0], 4 * tb + n, lane);
 #pragma unroll
         for (int i = 0; i < 2; ++i) dw1[i][n] = mfma6(av[i], b, dw1[i][n]);
         if (n & 1) __builtin_amdgcn_sched_barrier(0);
