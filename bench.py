@@ -1014,8 +1014,8 @@ def main_ppo(args, torch, dev):
         "value": samples / el, "unit": "samples/s", "n_gpus": 1, "steps": reps,
         "warmup": 1, "ms_per_step": el * 1e3, "higher_is_better": True, "scaling": "weak",
         "vs_baseline": None,
-        "dtype": "f16 MFMA first layer (f32 accumulate) / f16 hi/lo pair MFMA fused loss + backward "
-                 "+ weight gradients (f32 accumulate) / f32 torch Adam",
+        "dtype": "f16 MFMA first layer (f32 accumulate) / f32 fused loss + backward + weight gradients "
+                 "as bf16 triple MFMA products (f32 accumulate) / f32 torch Adam",
         "data": "synthetic: a buffer collected by the kernels from template maps, acted by "
                 "the learner's weights (the reference ActorCritic's orthogonal init)",
         "config": {"workload": "PPO update over a 5632 x 128 rollout buffer "

@@ -22,9 +22,12 @@
 // goes to HBM; a row-output kernel followed by batched products moved 4.2 KB
 // per row out and 3.5 KB back in.  Partial sums go to the workspace once per
 // workgroup and ppo_finish_kernel adds them in workgroup order
-// (deterministic).  Measured on a 180,224-row minibatch: 401 us with 18 us of
+// (deterministic).  Measured on a 180,224-row minibatch: 347 us with 18 us of
 // packing and reduction beside it, where the row-output kernel (float32 MFMA),
-// its batched products, reductions and copies took 860 us.
+// its batched products, reductions and copies took 860 us; 36 k cycles per
+// 32-row tile: the two backward product phases 9.1 k (MFMA-bound), the two
+// LayerNorms at the tile's ends 4.2 k, loss and dhy 3.2 k each, the others 2.1
+// to 2.5 k, waiting at the nine barriers 7.5 k.
 //
 // Products: v_mfma_f32_16x16x32_bf16 on three bfloat16 pieces of each operand,
 // x = x0 + x1 + x2, which hold float32's 24 bits at any magnitude: a row or a
@@ -72,7 +75,10 @@ constexpr int MAX_WGS = 256;  // one workgroup per CU
 // reads (8 rows per cycle) and the transposing reads (4 rows of 32 bytes) are
 // conflict-free
 constexpr int HS = H + 16, YS = HY + 16;
-constexpr int XS = H + 4, HYS = HY + 4;     // float rows
+// float rows; a head's hidden units (and an output's weights) are 68 apart, so
+// that the eight outputs of a row read distinct banks (64 apart they took
+// turns: 5.2 k of 38 k cycles of a tile in the loss phase, 3.6 k of 36 k now)
+constexpr int XS = H + 4, HP = 64 + 4, HYS = 3 * HP;
 constexpr float LN_EPS = 1e-5f;
 
 // weight fragments of the workspace (values): [tile][K step][piece][lane][8]
@@ -108,7 +114,7 @@ struct __align__(16) Lds {
   uint32_t in[R][16];                       // loss inputs (fetch_loss)
   float sum[3][R][16];                      // each thread's running output-gradient sum, statistic, max |dz1|
   float ln[4][H];                           // gamma1, beta1, gamma2, beta2
-  float b1[H], bh[HY], wf[8][64], bf[8];
+  float b1[H], bh[HY], wf[8][HP], bf[8];
   float mx[8];                              // per wavefront: max |dz1|
 };
 
@@ -171,37 +177,42 @@ __device__ __forceinline__ void put8(const float (&v)[8], uint16_t (&plane)[3][R
   for (int k = 0; k < 3; ++k) *reinterpret_cast<bf8*>(&plane[k][row][at]) = p[k];
 }
 
-// c += a b without the three products below 2^-25 of it
-__device__ __forceinline__ floatx4 mfma6(const bf8 (&a)[3], const bf8 (&b)[3], floatx4 c) {
-  c = __builtin_amdgcn_mfma_f32_16x16x32_bf16(a[2], b[0], c, 0, 0, 0);
-  c = __builtin_amdgcn_mfma_f32_16x16x32_bf16(a[0], b[2], c, 0, 0, 0);
-  c = __builtin_amdgcn_mfma_f32_16x16x32_bf16(a[1], b[1], c, 0, 0, 0);
-  c = __builtin_amdgcn_mfma_f32_16x16x32_bf16(a[1], b[0], c, 0, 0, 0);
-  c = __builtin_amdgcn_mfma_f32_16x16x32_bf16(a[0], b[1], c, 0, 0, 0);
-  return __builtin_amdgcn_mfma_f32_16x16x32_bf16(a[0], b[0], c, 0, 0, 0);
+// The six products of two operands' pieces, smallest first; the three left out
+// are below 2^-25 of the whole.
+constexpr int PA[6] = {2, 0, 1, 1, 0, 0}, PB[6] = {0, 2, 1, 0, 1, 0};
+
+__device__ __forceinline__ floatx4 mfma_bf(bf8 a, bf8 b, floatx4 c) {
+  return __builtin_amdgcn_mfma_f32_16x16x32_bf16(a, b, c, 0, 0, 0);
 }
 
-// The same with the leading products summed apart from the others (c[0], c[1]):
-// one rounding of the whole sum per step of 32 instead of six.
-__device__ __forceinline__ void mfma6(const bf8 (&a)[3], const bf8 (&b)[3], floatx4 (&c)[2]) {
-  c[1] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(a[2], b[0], c[1], 0, 0, 0);
-  c[1] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(a[0], b[2], c[1], 0, 0, 0);
-  c[0] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(a[0], b[0], c[0], 0, 0, 0);
-  c[1] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(a[1], b[1], c[1], 0, 0, 0);
-  c[1] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(a[1], b[0], c[1], 0, 0, 0);
-  c[1] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(a[0], b[1], c[1], 0, 0, 0);
+// c[i] += a[i] b for N tiles, product by product (N independent accumulators
+// between two uses of one)
+template <int N, int M>
+__device__ __forceinline__ void add_products(const bf8 (&a)[N][3], const bf8 (&b)[3], floatx4 (&c)[N][M], int n) {
+#pragma unroll
+  for (int k = 0; k < 6; ++k)
+#pragma unroll
+    for (int i = 0; i < N; ++i) c[i][n] = mfma_bf(a[i][PA[k]], b[PB[k]], c[i][n]);
 }
 
 // The pieces of eight consecutive features of a row.
-struct Pieces {
-  bf8 p[3];
-};
 template <int S>
-__device__ __forceinline__ Pieces ld_pieces(const uint16_t (&plane)[3][R][S], int row, int at) {
-  Pieces f;
+__device__ __forceinline__ void ld_pieces(bf8 (&f)[3], const uint16_t (&plane)[3][R][S], int row, int at) {
 #pragma unroll
-  for (int n = 0; n < 3; ++n) f.p[n] = ld8(&plane[n][row][at]);
-  return f;
+  for (int n = 0; n < 3; ++n) f[n] = ld8(&plane[n][row][at]);
+}
+
+// One K step of a data product: c[u] += a[u's tile] b[u's rows], the leading
+// product into c[u][0] and the others into c[u][1] (one rounding of the whole
+// sum per step of 32 instead of six).
+__device__ __forceinline__ void data_step(const bf8 (&a)[3], const bf8 (&b)[2][3], floatx4 (&c)[2][2]) {
+#pragma unroll
+  for (int k = 0; k < 6; ++k)
+#pragma unroll
+    for (int rt = 0; rt < 2; ++rt) {
+      floatx4& t = c[rt][k == 5 ? 0 : 1];
+      t = mfma_bf(a[PA[k]], b[rt][PB[k]], t);
+    }
 }
 
 // Sum of each of the eight values over the wavefront's four 16-lane rows;
@@ -429,9 +440,12 @@ __global__ __launch_bounds__(T) void ppo_step_kernel(const qqt_ppo_step_args a, 
     {
       floatx4 c[2][2] = {};                     // [row tile][leading | others]
 #pragma unroll
-      for (int k = 0; k < 4; ++k)
+      for (int k = 0; k < 4; ++k) {
+        bf8 b[2][3];
 #pragma unroll
-        for (int rt = 0; rt < 2; ++rt) mfma6(wz[k], ld_pieces(s.h1, 16 * rt + r16, 32 * k + 8 * q).p, c[rt]);
+        for (int rt = 0; rt < 2; ++rt) ld_pieces(b[rt], s.h1, 16 * rt + r16, 32 * k + 8 * q);
+        data_step(wz[k], b, c);
+      }
       const floatx4 b = *reinterpret_cast<const floatx4*>(&s.b1[16 * w + 4 * q]);
 #pragma unroll
       for (int rt = 0; rt < 2; ++rt)
@@ -462,11 +476,16 @@ __global__ __launch_bounds__(T) void ppo_step_kernel(const qqt_ppo_step_args a, 
       floatx4 c[3][2] = {};
 #pragma unroll
       for (int k = 0; k < 4; ++k) {
-        const Pieces b0 = ld_pieces(s.h2, 16 * tb + r16, 32 * k + 8 * q);
-        const Pieces b1 = ld_pieces(s.h2, 16 * (tb ^ 1) + r16, 32 * k + 8 * q);
-        mfma6(wy[k][0], b0.p, c[0]);
-        mfma6(wy[k][0], b1.p, c[1]);
-        mfma6(wy[k][1], b0.p, c[2]);
+        bf8 b[2][3];
+#pragma unroll
+        for (int u = 0; u < 2; ++u) ld_pieces(b[u], s.h2, 16 * (tb ^ u) + r16, 32 * k + 8 * q);
+#pragma unroll
+        for (int n = 0; n < 6; ++n)
+#pragma unroll
+          for (int u = 0; u < 3; ++u) {
+            floatx4& t = c[u][n == 5 ? 0 : 1];
+            t = mfma_bf(wy[k][u >> 1][PA[n]], b[u & 1][PB[n]], t);
+          }
       }
 #pragma unroll
       for (int u = 0; u < 3; ++u) {
@@ -475,7 +494,7 @@ __global__ __launch_bounds__(T) void ppo_step_kernel(const qqt_ppo_step_args a, 
         floatx4 v = (c[u][1] + c[u][0]) + b;
 #pragma unroll
         for (int i = 0; i < 4; ++i) v[i] = fmaxf(v[i], 0.0f);
-        *reinterpret_cast<floatx4*>(&s.hy[16 * rt + r16][16 * ft + 4 * q]) = v;
+        *reinterpret_cast<floatx4*>(&s.hy[16 * rt + r16][16 * ft + 4 * q + (HP - 64) * (ft >> 2)]) = v;
       }
       s.in[row][j] = lin;
     }
@@ -483,7 +502,7 @@ __global__ __launch_bounds__(T) void ppo_step_kernel(const qqt_ppo_step_args a, 
 
     // ---- outputs and loss: lanes 2o, 2o + 1 of a row's 16 hold output o
     {
-      const float* y = &s.hy[row][64 * grp + 32 * part];
+      const float* y = &s.hy[row][HP * grp + 32 * part];
       const float* wo = &s.wf[o][32 * part];
       floatx4 part4 = {0.0f, 0.0f, 0.0f, 0.0f};          // four short chains round less
 #pragma unroll
@@ -558,7 +577,7 @@ __global__ __launch_bounds__(T) void ppo_step_kernel(const qqt_ppo_step_args a, 
         const int r = 4 * w + rr;
         float dl[8];
         load8(&s.dl[r][0], dl);
-        const float y0 = s.hy[r][lane], y1 = s.hy[r][64 + lane], y2 = s.hy[r][128 + lane];
+        const float y0 = s.hy[r][lane], y1 = s.hy[r][HP + lane], y2 = s.hy[r][2 * HP + lane];
         float d0 = 0.0f;
 #pragma unroll
         for (int k = 0; k < 5; ++k) {
@@ -595,9 +614,12 @@ __global__ __launch_bounds__(T) void ppo_step_kernel(const qqt_ppo_step_args a, 
     {
       floatx4 c[2][2] = {};                     // [row tile][leading | others]
 #pragma unroll
-      for (int k = 0; k < 6; ++k)
+      for (int k = 0; k < 6; ++k) {
+        bf8 b[2][3];
 #pragma unroll
-        for (int rt = 0; rt < 2; ++rt) mfma6(wd[k], ld_pieces(s.dy, 16 * rt + r16, 32 * k + 8 * q).p, c[rt]);
+        for (int rt = 0; rt < 2; ++rt) ld_pieces(b[rt], s.dy, 16 * rt + r16, 32 * k + 8 * q);
+        data_step(wd[k], b, c);
+      }
 #pragma unroll
       for (int rt = 0; rt < 2; ++rt)
         *reinterpret_cast<floatx4*>(&s.ex[16 * rt + r16][16 * w + 4 * q]) = c[rt][1] + c[rt][0];
@@ -611,8 +633,7 @@ __global__ __launch_bounds__(T) void ppo_step_kernel(const qqt_ppo_step_args a, 
         bf8 b[3];
 #pragma unroll
         for (int m = 0; m < 3; ++m) b[m] = ld_rows<bf8, HS>(s.h2[m][0], 4 * tb + n, lane);
-#pragma unroll
-        for (int i = 0; i < 3; ++i) dwh[i][n] = mfma6(av[i], b, dwh[i][n]);
+        add_products(av, b, dwh, n);
         if (n & 1) __builtin_amdgcn_sched_barrier(0);
       }
     }
@@ -636,9 +657,12 @@ __global__ __launch_bounds__(T) void ppo_step_kernel(const qqt_ppo_step_args a, 
     {
       floatx4 c[2][2] = {};                     // [row tile][leading | others]
 #pragma unroll
-      for (int k = 0; k < 4; ++k)
+      for (int k = 0; k < 4; ++k) {
+        bf8 b[2][3];
 #pragma unroll
-        for (int rt = 0; rt < 2; ++rt) mfma6(wu[k], ld_pieces(s.dz, 16 * rt + r16, 32 * k + 8 * q).p, c[rt]);
+        for (int rt = 0; rt < 2; ++rt) ld_pieces(b[rt], s.dz, 16 * rt + r16, 32 * k + 8 * q);
+        data_step(wu[k], b, c);
+      }
 #pragma unroll
       for (int rt = 0; rt < 2; ++rt)
         *reinterpret_cast<floatx4*>(&s.ex[16 * rt + r16][16 * w + 4 * q]) = c[rt][1] + c[rt][0];
@@ -652,8 +676,7 @@ __global__ __launch_bounds__(T) void ppo_step_kernel(const qqt_ppo_step_args a, 
         bf8 b[3];
 #pragma unroll
         for (int m = 0; m < 3; ++m) b[m] = ld_rows<bf8, HS>(s.h1[m][0], 4 * tb + n, lane);
-#pragma unroll
-        for (int i = 0; i < 2; ++i) dw1[i][n] = mfma6(av[i], b, dw1[i][n]);
+        add_products(av, b, dw1, n);
         if (n & 1) __builtin_amdgcn_sched_barrier(0);
       }
     }
