@@ -103,13 +103,20 @@ class _Linear(torch.autograd.Function):
 
 
 def _seq_weight_grad(dy: torch.Tensor, x: torch.Tensor) -> torch.Tensor:
-    """`_weight_grad` for the recurrence's weights: chunks short enough that a
+    """`dy^T x` for the recurrence's weights: chunks short enough that a
     float32 sum within one is no longer than a frame's own product would be
     (error against float64 of dW_ih and dW_hh, 32 frames x 256 envs: chunks of
     256 rows 1.8e-7, of 1,024 2.6e-7, of 4,096 7.4e-7, frame by frame through
     nn.LSTM 2.0e-7; 12 x 37: chunks of 64 6.0e-7, of 256 1.0e-6, nn.LSTM
     6.2e-7), and at most a few hundred of them."""
-    return _weight_grad(dy, x, chunk=min(512, max(64, dy.shape[0] // 32)))
+    rows = dy.shape[0]
+    chunk = min(512, max(64, rows // 32))
+    c, n = rows // chunk, rows // chunk * chunk
+    if c < 2:
+        return dy.t() @ x
+    out = torch.bmm(dy[:n].reshape(c, chunk, -1).transpose(1, 2),
+                    x[:n].reshape(c, chunk, -1)).sum(0)
+    return out.addmm_(dy[n:].t(), x[n:]) if n < rows else out
 
 
 class _InputProduct(_Linear):
@@ -118,8 +125,8 @@ class _InputProduct(_Linear):
     that is larger than everything the recurrence adds (hidden outputs of 32
     frames x 256 envs against float64, mean of eight inputs: 1.37e-7 relative
     with one sum, 1.05e-7 with quarters, 1.06e-7 through nn.LSTM's own
-    kernels).  The input gradient sums eighths of its 512 gates: 12 x 37 frames 2.4e-7 in
-    quarters, 1.8e-7 through nn.LSTM."""
+    kernels).  The input gradient sums eighths of its 512 gates: 12 frames x
+    37 envs 2.0e-7, in quarters 2.4e-7, through nn.LSTM 1.8e-7."""
 
     @staticmethod
     def forward(ctx, x, w, b):
@@ -135,10 +142,8 @@ class _InputProduct(_Linear):
     def backward(ctx, dy):
         x, w = ctx.saved_tensors
         dy = dy.contiguous()
-        step = -(-w.shape[0] // 8)
-        dx = dy[:, :step] @ w[:step]
-        for k in range(step, w.shape[0], step):
-            dx = torch.addmm(dx, dy[:, k:k + step], w[k:k + step])
+        eighths = dy.reshape(-1, 8, w.shape[0] // 8).transpose(0, 1)
+        dx = torch.bmm(eighths, w.reshape(8, -1, w.shape[1])).sum(0)
         return dx, _seq_weight_grad(dy, x), dy.sum(0)
 
 
