@@ -29,8 +29,8 @@
 // row in two products.  Tiles of 256 columns (two workgroups per CU) read and
 // split dz1 twice as often, transposed both operands with VALU permutes and
 // had one step of loads in flight: a 180,224-row minibatch of scattered rows
-// took 335 us, now 294; with its rows cached 230, about the rate a library
-// float16 product of 8192^3 reaches on the same card (1.2 PFLOP/s: 180 us).
+// took 335 us, now 280; with its rows cached 231 (a library float16 product of
+// 8192^3 reaches 1.2 PFLOP/s on the same card: 180 us).
 
 #include <hip/hip_fp16.h>
 #include <hip/hip_runtime.h>
@@ -247,7 +247,7 @@ __device__ __forceinline__ void l1_grad_chunk(const qqt_l1_grad_args& a, Lds<NC>
 // slot's chunks in the workspace instead, which the wide tile would need, took
 // 232 us for 8,192 rows in four slots.)  The narrow tile is held to 128 registers
 // (7 go to scratch): two workgroups per CU take 45,056 rows in 17 slots in
-// 115 us, one (156 registers) in 134.
+// 114 us, one (156 registers) in 134.
 template <int NC, bool EDGE>
 __device__ __forceinline__ void l1_grad_slot(const qqt_l1_grad_args& a, Lds<NC>& s, int chunks,
                                              int chunk_rows, int ws_cols, int per_slot) {
@@ -328,10 +328,10 @@ __global__ __launch_bounds__(256) void l1_grad_reduce(const qqt_l1_grad_args a, 
 // The first layer's weight as the float16 MFMA B fragments the forward reads,
 // [tile][kblock][lane 16 q + r][16]: value i is row 16 tile + r, column
 // cols[64 kblock + 16 q + i], zero from k0 on.  A thread writes 16 bytes; a
-// launch moves 1.8 MB (1.2 read, 0.6 written) and is latency.  In its place
-// were an index, a fill, two copies and a conversion; with the column order of
-// dW0 (another index launch) folded into l1_grad_reduce, the gradients of an
-// 8192-row minibatch went 192 -> 159 us and of 180,224 rows 895 -> 866 us.
+// launch moves 1.8 MB (1.2 read, 0.6 written) and is latency (5 us).  In its
+// place were an index, a fill, two copies and a conversion; with the column
+// order of dW0 (another index launch) folded into l1_grad_reduce, 33 us of the
+// gradients of an 8192-row minibatch (192 -> 159) and 29 of 180,224 rows.
 __global__ __launch_bounds__(256) void w0_pack_kernel(const float* w, const int64_t* cols, int k0,
                                                       int kblocks, uint16_t* out) {
   const int i = blockIdx.x * 256 + threadIdx.x;           // 8 halves each
@@ -372,8 +372,8 @@ __host__ inline int pieces(int batch, int k0, int min_rows, int& rows) {
 // the narrow tile, walk its group's chunks and add as they go.  Below 512 rows a
 // chunk's partial tiles (1.3 MB out and back) cost what the shorter walk saves.
 // With the reduction, 2366 columns, in the documented workspace (one chunk per
-// slot, wide tile -> groups) and in the preferred one: 8,192 rows 134 -> 60 and
-// 32 us, 45,056 rows 142 -> 115 and 90 us.
+// slot, wide tile -> groups) and in the preferred one: 8,192 rows 134 -> 58 and
+// 32 us, 45,056 rows 142 -> 114 and 90 us.
 struct Plan {
   int chunks, rows, group;
 };

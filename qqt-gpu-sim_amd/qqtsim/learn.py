@@ -14,11 +14,15 @@ first-layer part of `mlp_act_kernel` (float16 MFMA, W0 rounded to float16
 as in acting, float32 accumulation; `qqt_mlp_act` with `z1_out`), its weight
 gradient `qqt_l1_grad` (float16 MFMA over the batch, dz1 split hi/lo after
 a power-of-two scale, float32 accumulation).  No input gradient is formed
-(the observation is data).  LayerNorm, the 128-wide layers and the heads
-run as torch ops on the same device (about 8 % of the FLOPs); their weight
-gradients, whose reduction runs over the whole minibatch, are batched
-products over row chunks (a single batch-long reduction lands on a few
-workgroups).
+(the observation is data).
+
+Two paths lead through it.  `ppo_grads`, which `ppo_update` takes, runs a
+minibatch's loss and everything above the first layer, weight gradients
+included, in one kernel (`qqt_ppo_step`).  `forward` / `evaluate` with
+autograd keep the reference's own calls: there LayerNorm, the 128-wide layers
+and the heads are torch ops (about 8 % of the FLOPs), and their weight
+gradients, whose reduction runs over the whole minibatch, batched products over
+row chunks (a single batch-long reduction lands on a few workgroups).
 
 `ppo_update` is the reference's update loop (train/ppo.py:364-437) over a
 device rollout buffer, with the GAE scan on `qqt_gae`; for the lstm arch

@@ -21,7 +21,7 @@ def _case(b, seed, dev, outliers):
                        torch.multinomial(bm.float().cpu(), 1, generator=g)[:, 0]], 1).to(dev)
     f = lambda s: (s * torch.randn(b, generator=g)).to(dev)  # noqa: E731
     old_logp, adv, ret, old_val = f(0.3) - 1.5, f(1.0), f(1.0), f(1.0)
-    if outliers:                 # the running scale of the gradients falls in a later tile
+    if outliers:                 # rows whose gradients are orders of magnitude above the others'
         adv[b // 2], ret[-1] = 3e4, 1e5
     return obs, mm, bm, act, old_logp, adv, ret, old_val
 
